@@ -438,10 +438,14 @@ __device__ __forceinline__ void cast_block(const AttnArgs &a, f32x16 &s) {
   }
   if (a.flags & ATT_RND_SCORE) round_block(s);
 }
-// query block qb's key chunks (bf16 softmax statistics)
+// query block qb's 32-key blocks (the last one partial when S is no multiple
+// of 32) and key chunks (bf16 softmax statistics)
+__device__ __forceinline__ int stat_blocks(const AttnArgs &a, int qb) {
+  const int nb = (a.S + 31) / 32;
+  return a.causal ? min((qb + 1) * 4, nb) : nb;
+}
 __device__ __forceinline__ int stat_chunks(const AttnArgs &a, int qb) {
-  const int nb = a.causal ? (qb + 1) * 4 : a.S / 32;
-  return (nb + a.ckb - 1) / a.ckb;
+  return (stat_blocks(a, qb) + a.ckb - 1) / a.ckb;
 }
 
 // x0, x1 rounded to bf16 (round to nearest even) with one packed
@@ -473,9 +477,20 @@ __device__ __forceinline__ void round_bf16x2(float &x0, float &x1) {
 // midpoint (a midpoint times l has a set bit below e's last) and lies at
 // least 2^-17 (relative) from one, beyond the 2^-23 the product can stray
 // from the correctly rounded quotient: both round to the same bf16 value.
-template <int NW, bool XF = false, bool SMX = false>
+//
+// RAG: S of any length.  The last query block and the last 32-key block may
+// be partial: keys past S come in as zeros (past the end of the resources)
+// and are masked (causal: no stored query sees them), queries past S repeat
+// the last query's loads and store nothing.  The weights of the fp32 softmax
+// then enter the P V MFMAs as a pair of bf16 values, p = hi + lo to 2^-17
+// (two MFMAs per fragment): such lengths ran on the unfused kernels, whose
+// weights are fp32, and keep that accuracy.  Batch 2, S = 1000, 32 / 8 heads:
+// the fp8 attention block 6811 us unfused, 241 us with this kernel (and the
+// Qwen3 prefill layer of 1500 tokens 9387 -> 388 us).
+template <int NW, bool XF = false, bool SMX = false, bool RAG = false>
 __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   static_assert(!SMX || XF, "the bf16 softmax follows the score cast points");
+  constexpr bool SPLIT = RAG && !SMX;  // weights as hi + lo
   constexpr int AQW = 32 * NW;  // queries per workgroup
   constexpr int TB = 32 * AD * 2;  // one 32-key K or V tile
   // one array per operand: a slot is a constant offset, so one address
@@ -495,7 +510,7 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
 
   // work item order as in attention_causal_body: contiguous ranges per XCD,
   // longest query blocks of a KV head first
-  const int nqb = a.S / AQW;
+  const int nqb = RAG ? (a.S + AQW - 1) / AQW : a.S / AQW;
   const int rep = a.Hq / a.Hkv;
   const int per_kv = rep * nqb;
   const int nwg = a.B * a.Hkv * per_kv;
@@ -519,13 +534,14 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
 
   const int wq0 = q0 + wave * 32;
   const int qrow = wq0 + l32;
+  const int qld = RAG ? min(qrow, a.S - 1) : qrow;  // the row this lane loads
   // SMX: this query's max score, bf16 weight sum and RN(1 / sum), from the
   // statistics of its query block's key chunks (the sums added in chunk
   // order)
   float mx = 0.f, lb = 1.f, rlb = 1.f;
   if constexpr (SMX) {
     const int64_t nq = (int64_t)a.B * a.Hq * a.S;
-    const float *st = a.rowstat + ((int64_t)b * a.Hq + h) * a.S + qrow;
+    const float *st = a.rowstat + ((int64_t)b * a.Hq + h) * a.S + qld;
     const int nc = stat_chunks(a, qb);
     mx = st[0];
     float tot = st[a.nch * nq];
@@ -539,7 +555,7 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   bf16x8_t qf[AD / 16];
 #pragma unroll
   for (int kk = 0; kk < AD / 16; ++kk)
-    qf[kk] = *reinterpret_cast<const bf16x8_t *>(qp + (int64_t)qrow * a.q_ss + kk * 16 + lhi * 8);
+    qf[kk] = *reinterpret_cast<const bf16x8_t *>(qp + (int64_t)qld * a.q_ss + kk * 16 + lhi * 8);
 
   f32x16 acc_o[4];
 #pragma unroll
@@ -552,8 +568,9 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   const float sl2 = XF ? 1.44269504088896340736f : a.scale * 1.44269504088896340736f;
 
   // key blocks: the workgroup's (the last wave's causal extent) and this wave's
-  const int nb_wg = a.causal ? (q0 + AQW) / 32 : a.S / 32;
-  const int nb_w = a.causal ? wq0 / 32 + 1 : a.S / 32;
+  const int nb_s = RAG ? (a.S + 31) / 32 : a.S / 32;  // the sequence's
+  const int nb_wg = a.causal ? (RAG ? min((q0 + AQW) / 32, nb_s) : (q0 + AQW) / 32) : nb_s;
+  const int nb_w = a.causal ? (RAG ? min(wq0 / 32 + 1, nb_wg) : wq0 / 32 + 1) : nb_s;
   // iterations 1 .. U-1 run for every wave with no mask: causal, block j + 1
   // lies below the first wave's diagonal block q0 / 32
   const int U = a.causal ? q0 / 32 : nb_wg - 1;
@@ -616,8 +633,10 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s, 0, 0, 0);
     }
   };
-  // O^T += V^T P^T for one block (P as two 16-key bf16 fragments)
-  auto pv = [&](const uint8_t *Vt, const bf16x8_t (&pf)[2]) __attribute__((always_inline)) {
+  // O^T += V^T P^T for one block (P as two 16-key bf16 fragments, SPLIT: and
+  // two of the rest of each weight)
+  constexpr int NP = SPLIT ? 4 : 2;
+  auto pv = [&](const uint8_t *Vt, const bf16x8_t (&pf)[NP]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -629,10 +648,11 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
         const bf16x8_t vf = __builtin_shufflevector(__builtin_bit_cast(bf16x4_t, v[0]),
                                                     __builtin_bit_cast(bf16x4_t, v[1]), 0, 1, 2, 3, 4, 5, 6, 7);
         acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[j], acc_o[dt], 0, 0, 0);
+        if constexpr (SPLIT) acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[2 + j], acc_o[dt], 0, 0, 0);
       }
   };
   // p = 2^(s c - m) of one block -> bf16 fragments; returns this lane's sum
-  auto expblock = [&](const f32x16 &s, bf16x8_t (&pf)[2]) __attribute__((always_inline)) {
+  auto expblock = [&](const f32x16 &s, bf16x8_t (&pf)[NP]) __attribute__((always_inline)) {
     float ps0 = 0.f, ps1 = 0.f;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -641,13 +661,14 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + e], sl2, -m_run));
         if (e & 1) ps1 += p; else ps0 += p;
         pf[j][e] = (__bf16)p;
+        if constexpr (SPLIT) pf[2 + j][e] = (__bf16)(p - (float)pf[j][e]);
       }
     return ps0 + ps1;
   };
   // the softmax of one block (scores s, key block kb); with MASK, keys past
   // klim (the query itself when causal, else the last key) get p = 0
   const int klim = a.causal ? qrow : a.S - 1;
-  auto softmax = [&](f32x16 &s, bf16x8_t (&pf)[2], int kb, auto masktag) __attribute__((always_inline)) {
+  auto softmax = [&](f32x16 &s, bf16x8_t (&pf)[NP], int kb, auto masktag) __attribute__((always_inline)) {
     if constexpr (XF) cast_block(a, s);
     if constexpr (decltype(masktag)::value) {
       // element r holds key kb * 32 + 4 lhi + (8 (r / 4) + r % 4)
@@ -694,9 +715,9 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   };
 
   f32x16 sA, sB;
-  bf16x8_t pA[2], pB[2];
+  bf16x8_t pA[NP], pB[NP];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < NP; ++j)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       pA[j][e] = (__bf16)0.f;
@@ -706,8 +727,8 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   // Iteration j (SL = j mod 4).  Register sets alternate with the parity of
   // j: s_cur holds block j's scores, s_nxt receives block j + 1's; p_cur
   // receives block j's P, p_prev holds block j - 1's.
-  auto iter = [&](auto sl, auto gen, int j, f32x16 &s_cur, f32x16 &s_nxt, bf16x8_t (&p_prev)[2],
-                  bf16x8_t (&p_cur)[2]) __attribute__((always_inline)) {
+  auto iter = [&](auto sl, auto gen, int j, f32x16 &s_cur, f32x16 &s_nxt, bf16x8_t (&p_prev)[NP],
+                  bf16x8_t (&p_cur)[NP]) __attribute__((always_inline)) {
     constexpr int SL = decltype(sl)::value;
     constexpr bool GEN = decltype(gen)::value;
     const uint8_t *kn = kslot(SlotTag<SL + 1>{});
@@ -722,7 +743,7 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
       __builtin_amdgcn_sched_group_barrier(0x100, 24, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
+      for (int i = 0; i < (SPLIT ? 24 : 16); ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
       }
@@ -792,6 +813,7 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   // normalise (the weights of the bf16 softmax are normalised already) and
   // store
   const float inv_l = SMX ? 1.0f : 1.0f / (l_run + __shfl_xor(l_run, 32, 64));
+  if (RAG && qrow >= a.S) return;
   uint16_t *orow = op + (int64_t)qrow * a.o_ss;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -812,6 +834,16 @@ extern "C" __global__ __launch_bounds__(256, 2) void nk_attention_causal_d128_sp
 }
 extern "C" __global__ __launch_bounds__(256, 2) void nk_attention_causal_d128_sp_xf_bf16(AttnArgs a) {
   attention_sp_body<4, true, true>(a);
+}
+// sequence lengths that are no multiple of 128
+extern "C" __global__ __launch_bounds__(256, 2) void nk_attention_causal_d128_sp_rag(AttnArgs a) {
+  attention_sp_body<4, false, false, true>(a);
+}
+extern "C" __global__ __launch_bounds__(256, 2) void nk_attention_causal_d128_sp_rag_xf(AttnArgs a) {
+  attention_sp_body<4, true, false, true>(a);
+}
+extern "C" __global__ __launch_bounds__(256, 2) void nk_attention_causal_d128_sp_rag_xf_bf16(AttnArgs a) {
+  attention_sp_body<4, true, true, true>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -840,7 +872,7 @@ __device__ __forceinline__ void attention_rowstat_body(const AttnArgs &a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31, lhi = lane >> 5;
-  const int nqb = a.S / 128, rep = a.Hq / a.Hkv;
+  const int nqb = (a.S + 127) / 128, rep = a.Hq / a.Hkv;
 
   int per_bg = 0;  // work items of one (batch, KV head)
   for (int qb = 0; qb < nqb; ++qb) per_bg += stat_chunks(a, qb);
@@ -864,11 +896,14 @@ __device__ __forceinline__ void attention_rowstat_body(const AttnArgs &a) {
   // block holding its own queries (causal); never empty, as a causal
   // chunk starts at or before the query block's first key block
   const int wq0 = qb * 128 + wave * 32, qrow = wq0 + l32;
+  // a query past the last (S no multiple of 128) repeats the last one's
+  // loads and stores nothing
+  const bool qin = qrow < a.S;
+  const int qld = qin ? qrow : a.S - 1;
+  const int klim = a.causal ? qrow : a.S - 1;  // this query's last key
   const int kb0 = c * a.ckb;
-  int kb1 = min(kb0 + a.ckb, a.causal ? (qb + 1) * 4 : a.S / 32);
-  if (a.causal) kb1 = min(kb1, wq0 / 32 + 1);
-
-  const int kb1_wg = min(kb0 + a.ckb, a.causal ? (qb + 1) * 4 : a.S / 32);  // the workgroup's blocks
+  const int kb1_wg = min(kb0 + a.ckb, stat_blocks(a, qb));  // the workgroup's blocks
+  const int kb1 = a.causal ? min(kb1_wg, wq0 / 32 + 1) : kb1_wg;
   const uint16_t *qp = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
   const uint16_t *kp = a.k + (int64_t)b * a.k_sb + (int64_t)g * a.k_sh;
   const i32x4_t rk = rsrc_words(kp, (int64_t)a.S * a.k_ss * 2);
@@ -876,7 +911,7 @@ __device__ __forceinline__ void attention_rowstat_body(const AttnArgs &a) {
   constexpr int TB = 32 * AD * 2;  // one K tile
   __shared__ __attribute__((aligned(1024))) uint8_t KT[4 * TB];
   const int64_t nq = (int64_t)a.B * a.Hq * a.S;
-  float *st = a.rowstat + ((int64_t)b * a.Hq + h) * a.S + qrow;
+  float *st = a.rowstat + ((int64_t)b * a.Hq + h) * a.S + qld;
   bf16x8_t qf[AD / 16];  // loaded once the first moves are out
   float mx = 0.f;        // SUM: the query's max score, likewise
 
@@ -907,9 +942,10 @@ __device__ __forceinline__ void attention_rowstat_body(const AttnArgs &a) {
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t *>(Kt + koff(kk)), qf[kk], s,
                                                   0, 0, 0);
     if constexpr (SUM) cast_block(a, s);
-    if (a.causal && kb == wq0 / 32) {
+    // the block holding this wave's queries, or the partial last block
+    if (a.causal ? kb == wq0 / 32 : kb * 32 + 32 > a.S) {
       // element r holds key kb * 32 + 4 lhi + (8 (r / 4) + r % 4)
-      const int t = qrow - kb * 32 - lhi * 4;
+      const int t = klim - kb * 32 - lhi * 4;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = ((r >> 2) * 8 + (r & 3)) > t ? -INFINITY : s[r];
     }
@@ -947,7 +983,7 @@ __device__ __forceinline__ void attention_rowstat_body(const AttnArgs &a) {
   // own inside the loop
 #pragma unroll
   for (int kk = 0; kk < AD / 16; ++kk)
-    qf[kk] = *reinterpret_cast<const bf16x8_t *>(qp + (int64_t)qrow * a.q_ss + kk * 16 + lhi * 8);
+    qf[kk] = *reinterpret_cast<const bf16x8_t *>(qp + (int64_t)qld * a.q_ss + kk * 16 + lhi * 8);
   if constexpr (SUM) {
     const int nc = stat_chunks(a, qb);
     mx = st[0];
@@ -967,10 +1003,10 @@ __device__ __forceinline__ void attention_rowstat_body(const AttnArgs &a) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no move outlives the workgroup
   if constexpr (SUM) {
     acc += __shfl_xor(acc, 32, 64);
-    if (lhi == 0) st[(a.nch + c) * nq] = acc;
+    if (lhi == 0 && qin) st[(a.nch + c) * nq] = acc;
   } else {
     acc = fmaxf(acc, __shfl_xor(acc, 32, 64));
-    if (lhi == 0) st[c * nq] = cast_score(a, acc);
+    if (lhi == 0 && qin) st[c * nq] = cast_score(a, acc);
   }
 }
 extern "C" __global__ __launch_bounds__(256) void nk_attention_rowmax_d128(AttnArgs a) {

@@ -1010,11 +1010,12 @@ def divide_rounds_as_multiply(div: float) -> bool:
 
 def attention_stat_chunks(S: int, causal: bool = True):
     """Key chunks of the bf16 softmax's row statistics: (32-key blocks per
-    chunk, most chunks of a query block, chunks summed over the S / 128
-    query blocks).  Chunks of 512 keys, or of S / 8 rounded up to 128 keys
+    chunk, most chunks of a query block, chunks summed over the query blocks
+    of 128).  Chunks of 512 keys, or of S / 8 rounded up to 128 keys
     when S passes 4096, so a row has at most 8."""
     ckb = 4 * max(4, -(-S // 1024))
-    per_qb = [-(-((qb + 1) * 4 if causal else S // 32) // ckb) for qb in range(S // 128)]
+    nb = -(-S // 32)
+    per_qb = [-(-(min((qb + 1) * 4, nb) if causal else nb) // ckb) for qb in range(-(-S // 128))]
     return ckb, max(per_qb), sum(per_qb)
 
 
@@ -1027,7 +1028,7 @@ def attention_rowstat_bytes(B: int, S: int, Hq: int, causal: bool = True) -> int
 def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq: int, Hkv: int,
               D: int, scale: float, strides: dict, causal: bool = True, waves: int = None,
               key_block: int = None, ring: bool = None, score_flags: int = 0,
-              divisor: float = None, rowstat_ptr: int = 0):
+              divisor: float = None, rowstat_ptr: int = 0, ragged: bool = False):
     """Flash-style attention over bf16 q (B, S, Hq, D), k / v (B, S, Hkv, D) and
     o (B, S, Hq, D), each addressed by element strides {"q": (sb, ss, sh), ...}
     with the head dim contiguous.  KV head of query head h is h // (Hq // Hkv).
@@ -1035,6 +1036,9 @@ def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq
     ``key_block`` (64 or 32) keys per step.  Variants: (4, 64), (8, 64) and
     (4, 32), the last with three workgroups per CU; ``ring`` selects the
     software-pipelined (4, 32) kernel over a four-slot K / V ring.
+    ``ragged`` selects that kernel's form for any S (partial last blocks of
+    queries and keys, the fp32 softmax's weights kept to 2^-17 as two bf16
+    parts); every other form needs S to be a multiple of 128.
 
     ``score_flags`` (ATT_*) give each score the traced code's cast points
     before the softmax: ATT_RND_PROD rounds q.k to bf16, ATT_DIVIDE divides
@@ -1052,7 +1056,7 @@ def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq
     list of three launches instead of one launch."""
     if D != 128:
         raise LaunchError(f"attention kernel is built for head_dim 128, got {D}")
-    if S % 128 or S <= 0:
+    if S <= 0 or (S % 128 and not ragged):
         raise LaunchError(f"attention needs the sequence length to be a multiple of 128, got {S}")
     if Hq % Hkv:
         raise LaunchError("query heads must be a multiple of KV heads")
@@ -1065,7 +1069,8 @@ def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq
             raise LaunchError("attention operands must be 16-byte aligned")
     if not scale > 0:
         raise LaunchError("attention kernel needs a positive score scale")
-    if S * max(strides["k"][1], strides["v"][1], 128) * 2 >= 2**31:
+    # (K / V moves address whole 32-key blocks with 32-bit offsets)
+    if -(-S // 32) * 32 * max(strides["k"][1], strides["v"][1], 128) * 2 >= 2**31:
         raise LaunchError("attention K / V rows of one sequence must span less than 2 GiB")
     if score_flags & ~(ATT_RND_PROD | ATT_RND_SCORE | ATT_SOFTMAX_BF16 | ATT_DIVIDE):
         raise LaunchError(f"unknown attention score flags {score_flags:#x}")
@@ -1109,13 +1114,15 @@ def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq
         (waves, key_block))
     if suffix is None:
         raise LaunchError(f"no attention variant with {waves} waves and {key_block}-key blocks")
-    if S % (32 * waves):
+    if ragged and (waves, ring) != (4, True):
+        raise LaunchError("attention over any length exists on the 4-wave ring kernel only")
+    if S % (32 * waves) and not ragged:
         raise LaunchError(f"attention with {waves} waves needs S to be a multiple of {32 * waves}")
-    nblocks = B * Hq * (S // (32 * waves))
+    nblocks = B * Hq * -(-S // (32 * waves))
     if nblocks >= 2**31:
         raise LaunchError("attention grid too large")
     flops = 4 * B * Hq * S * S * D // (2 if causal else 1)
-    sym = "nk_attention_causal_d128" + suffix + ("_xf" if score_flags else "")
+    sym = "nk_attention_causal_d128" + suffix + ("_rag" if ragged else "") + ("_xf" if score_flags else "")
     if smx_bf16:
         qk_bytes = (B * S * Hq * D + B * S * Hkv * D) * 2
         stat = 4 * nch * B * Hq * S
