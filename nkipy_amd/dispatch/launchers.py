@@ -261,8 +261,10 @@ GEMM_VEC = 8
 GEMM_RND_BIAS = 16
 GEMM_RND_RESID = 32
 GEMM_ROWS16 = 64
+GEMV_OUT4 = 128
 GEMM_BM = 256
 GEMM_BN = 256
+GEMM128_GROUP_M = 8  # tile rows per group of the 128-tile kernels' walk
 
 
 def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: str,
@@ -270,7 +272,8 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
          bias_ptr: int = 0, scale_ptr: int = 0, resid_ptr: int = 0,
          up_ptr: int = 0, up_scale_ptr: int = 0, pingpong: bool = None,
          round_before_bias: bool = False, round_before_resid: bool = False,
-         rope: GemmRope = None, stage64: bool = None, staged: bool = None) -> Launch:
+         rope: GemmRope = None, stage64: bool = None, staged: bool = None, tile: int = GEMM_BM,
+         kh: bool = None) -> Launch:
     """C[M, N] = A[M, K] @ B (+ epilogue) on bf16 MFMA, fp32 accumulation.
 
     ``layout`` "nn": B is K x N row-major (ldb >= N); "nt": B is N x K
@@ -291,7 +294,9 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
     (whole 128-byte lines per global read).  ``staged``
     (default: wherever it applies, i.e. 64-deep stages and a bf16 output in
     aligned 16-byte row chunks) writes the output tile through LDS so that
-    every global store covers whole lines.
+    every global store covers whole lines.  ``tile`` 128 selects the kernels
+    of 128 x 128 output tiles (gemm128.hip; no fp8 NN form, none of the other
+    options), ``kh`` their eight-wave form (default: at most 256 tiles).
     """
     if layout not in ("nn", "nt"):
         raise LaunchError(f"unknown GEMM layout {layout}")
@@ -329,8 +334,12 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
         raise LaunchError("SwiGLU with fp8 weights needs scales for both weights")
     if swiglu and (bias_ptr or resid_ptr or c_dtype != dt.bfloat16):
         raise LaunchError("the SwiGLU epilogue writes bf16 without bias / residual")
-    bn = GEMM_BN // 2 if swiglu else GEMM_BN
-    tiles_m = -(-M // GEMM_BM)
+    if tile not in (128, GEMM_BM):
+        raise LaunchError(f"GEMM output tiles are 128 or {GEMM_BM} wide, got {tile}")
+    if tile == 128 and ((fp8 and layout == "nn") or pingpong is not None or stage64 is not None or staged is not None):
+        raise LaunchError("the 128-tile GEMM has no fp8 NN form and no kernel options")
+    bn = tile // 2 if swiglu else tile
+    tiles_m = -(-M // tile)
     tiles_n = -(-N // bn)
     if tiles_m * tiles_n >= 2**31:
         raise LaunchError("GEMM grid too large")
@@ -371,6 +380,16 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
         args.rope_nq, args.rope_nk = rope.nq, rope.nk
     btag = "e4m3" if fp8 else "bf16"
     ctag = "bf16" if c_dtype == dt.bfloat16 else "f32"
+    n_mm = 2 if swiglu else 1
+    nbytes = M * K * 2 + n_mm * N * K * b_dtype.itemsize + M * N * c_dtype.itemsize
+    if tile == 128:
+        args.group_m = GEMM128_GROUP_M
+        symbol = (f"nk_gemm128_swiglu_{layout}_{btag}_bf16" if swiglu else
+                  f"nk_gemm128_{layout}_{btag}_{ctag}" + ("_rope" if rope is not None else ""))
+        kh = kh if kh is not None else tiles_m * tiles_n <= 256
+        symbol += "_kh" if kh else ""
+        return Launch("gemm128", symbol, (tiles_m * tiles_n, 1, 1), (512 if kh else 256, 1, 1), args, bytes=nbytes,
+                      flops=2 * M * N * K * n_mm)
     has_pp = not (fp8 and layout == "nn")
     if pingpong is None:
         pingpong = has_pp
@@ -396,12 +415,11 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
                           "chunks (a residual added after the bf16 rounding; 16-byte aligned rotary outputs)")
     if staged:
         symbol += "_r16"  # the output tile staged through LDS
-    n_mm = 2 if swiglu else 1
-    nbytes = M * K * 2 + n_mm * N * K * b_dtype.itemsize + M * N * c_dtype.itemsize
     return Launch("gemm", symbol, (tiles_m * tiles_n, 1, 1), (512 if pingpong else 256, 1, 1), args,
                   bytes=nbytes, flops=2 * M * N * K * n_mm)
 
 
+REDUCE4_MIN = 1 << 17
 SPLITK_TARGET_WGS = 256  # one 8-wave GEMM workgroup per CU
 
 
@@ -421,14 +439,54 @@ def gemm_splitk_split(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = 
     return -(-K // kc), kc
 
 
-def gemm_splitk_useful(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = False) -> bool:
-    """Whether the K-range form beats one K loop per tile: up to 64 rows
-    whenever it splits; up to 256 rows only when the tiles leave most CUs
-    idle (at most 32 tiles) -- 512 or more rows, or 256 rows of a 14336-wide
-    projection, measured slower split."""
-    if M > GEMM_BM or (M > 64 and -(-N // GEMM_BN) > 32):
-        return False
-    return gemm_splitk_split(M, N, K, swiglu, fp8)[0] > 1
+# Times of the GEMM forms, us per 1000 k of a round of workgroups (measured
+# cold, 24 to 3000 rows of 4096 / 6144 / 12288 / 14336-wide projections): a
+# round of 256 workgroups of 256 x 256 tiles; at most 256 workgroups of 128 x
+# 128 tiles in the eight-wave form; 512 of them in the four-wave form, two per
+# CU, in half rounds.  By weights: fp8 NT, bf16 NT, bf16 NN.
+_GEMM_US = {("nt", True): (20.3, 6.6, 14.6), ("nt", False): (23.5, 8.4, 17.2), ("nn", False): (20.0, 9.2, 16.5)}
+_GEMM_FIXED_US = 6.0      # launch, prologue, epilogue
+_GEMM_STREAM = 4.5e6      # weight bytes per us a short product streams at
+_PLANES_RATE = 5.0e6      # partial-sum bytes per us, written and read again
+GEMM128_MAX_M = 8192      # rows past which the 256 x 256 tiles fill the part at every width in use
+GEMM128_MAX_RANGES = 16
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = False,
+              ranges: bool = True) -> Tuple[int, int, int]:
+    """(tile, K ranges, k per range) of the fastest GEMM form by the table
+    above: the 256 x 256 tiles where they fill whole rounds (4096 rows of a
+    12288-wide projection), the 128 x 128 tiles where the large ones leave CUs
+    idle or padded (fp8, K 4096: 1000 x 6144 58 against 86 us, 1000 x 4096 37
+    against 85), and those over K ranges where they still do (300 x 4096 x
+    14336 fp8: 61 us in two ranges, 101 in one, 274 on the large tiles; 24
+    rows 24 us in eight ranges).  Ranges cost their fp32 planes written and
+    read once, and a second launch.  ``ranges`` False: one K loop per tile."""
+    if fp8 and layout == "nn":
+        return GEMM_BM, 1, K
+    c256, ckh, c128 = _GEMM_US[(layout, fp8)]
+    n_mm = 2 if swiglu else 1
+    stream = n_mm * N * K * (1 if fp8 else 2) / _GEMM_STREAM
+    tiles256 = -(-M // 256) * -(-(N * n_mm) // 256)
+    best = (max(stream, -(-tiles256 // 256) * c256 * K / 1000), (GEMM_BM, 1, K))
+    if M > GEMM128_MAX_M:
+        return best[1]
+    for want in range(1, (GEMM128_MAX_RANGES if ranges else 1) + 1):
+        kc = -(-(-(-K // want)) // 64) * 64
+        ks = -(-K // kc)
+        if ks != want:
+            continue
+        # a SwiGLU pair in ranges runs as two launches, gate and up
+        wgs = -(-M // 128) * (-(-N // 64) if swiglu and ks == 1 else -(-N // 128)) * ks
+        us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
+        if ks > 1:
+            planes = 4 * ks * M * N * n_mm
+            if planes > 1 << 28:
+                continue
+            us = n_mm * (max(us, stream / n_mm) + _GEMM_FIXED_US) + 2 * planes / _PLANES_RATE
+        best = min(best, (max(us, stream), (128, ks, kc)))
+    return best[1]
 
 
 def gemm_splitk_workspace_bytes(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = False) -> int:
@@ -439,13 +497,17 @@ def gemm_splitk_workspace_bytes(M: int, N: int, K: int, swiglu: bool = False, fp
 def gemm_splitk(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: str, b_dtype, c_dtype,
                 ws_ptr: int, lda: int = None, ldb: int = None, ldc: int = None, bias_ptr: int = 0,
                 scale_ptr: int = 0, resid_ptr: int = 0, up_ptr: int = 0, up_scale_ptr: int = 0,
-                round_before_bias: bool = False, round_before_resid: bool = False) -> List[Launch]:
-    """The operation of :func:`gemm` (no rotary form) for few rows: the MFMA
-    kernels over K ranges (grid y) into fp32 partial planes in the workspace
+                round_before_bias: bool = False, round_before_resid: bool = False,
+                split: Tuple[int, int] = None, kh: bool = None) -> List[Launch]:
+    """The operation of :func:`gemm` (no rotary form) for few rows: the
+    128-tile kernels over K ranges (grid y) into fp32 partial planes in the workspace
     at ``ws_ptr`` (``gemm_splitk_workspace_bytes``; the SwiGLU form runs the
     gate and the up weights into two sets of planes), then the reduction of
     :func:`gemv` adds the ranges in order and applies the epilogue.  bf16 NN,
-    bf16 NT and fp8 NT weights."""
+    bf16 NT and fp8 NT weights.  ``split`` = (ranges, k per range, a multiple
+    of 64) in place of :func:`gemm_splitk_split` (the workspace then holds 4 *
+    ranges * M * N bytes, twice that for SwiGLU); ``kh`` as for
+    :func:`gemm`."""
     if layout not in ("nn", "nt"):
         raise LaunchError(f"unknown GEMM layout {layout}")
     b_dtype, c_dtype = dt.canonical(b_dtype), dt.canonical(c_dtype)
@@ -470,19 +532,24 @@ def gemm_splitk(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, l
         raise LaunchError("the SwiGLU epilogue writes bf16 without bias / residual")
     if fp8 and not scale_ptr:
         raise LaunchError("fp8 weights need per-column scales")
-    ks, kc = gemm_splitk_split(M, N, K, swiglu, fp8)
+    ks, kc = gemm_splitk_split(M, N, K, swiglu, fp8) if split is None else split
+    if kc % 64 or kc <= 0 or ks != -(-K // kc):
+        raise LaunchError(f"K ranges must be multiples of 64 that cover K = {K}, got {ks} of {kc}")
     plane = M * N
     launches = []
     for i, bp in enumerate([b_ptr] + ([up_ptr] if swiglu else [])):
         # the operand checks of gemm(); fp32 partial sums, no epilogue
         part = gemm(a_ptr, bp, ws_ptr + 4 * i * ks * plane, M, N, K, layout=layout, b_dtype=b_dtype,
-                    c_dtype=dt.float32, lda=lda, ldb=ldb, ldc=N, pingpong=True,
-                    scale_ptr=1 if fp8 else 0)
+                    c_dtype=dt.float32, lda=lda, ldb=ldb, ldc=N,
+                    scale_ptr=1 if fp8 else 0, tile=128, kh=False)
         args = part.args
         args.scale0 = None
         args.flags &= GEMM_VEC
         args.ksplit, args.kc = ks, kc
-        launches.append(Launch("gemm", part.symbol + "_splitk", (part.grid[0], ks, 1), part.block, args,
+        symbol, block = part.symbol + "_splitk", part.block
+        if kh if kh is not None else part.grid[0] * ks <= 256:
+            symbol, block = symbol.replace("gemm128", "gemm8k"), (512, 1, 1)
+        launches.append(Launch(part.module, symbol, (part.grid[0], ks, 1), block, args,
                                bytes=M * K * 2 + N * K * b_dtype.itemsize + 4 * ks * plane,
                                flops=2 * M * N * K))
     flags = (GEMM_BIAS if bias_ptr else 0) | (GEMM_SCALE if scale_ptr else 0) | (GEMM_RESID if resid_ptr else 0)
@@ -492,11 +559,26 @@ def gemm_splitk(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, l
         flags |= GEMM_RND_RESID
     out = GemvArgs(a_ptr, b_ptr, up_ptr or None, c_ptr, bias_ptr or None, scale_ptr or None,
                    up_scale_ptr or None, resid_ptr or None, ws_ptr, M, N, K, lda, ldb, ldc, ks, kc, flags, 0)
-    ctag = "bf16" if c_dtype == dt.bfloat16 else "f32"
-    sw = "_swiglu" if swiglu else ""
-    launches.append(Launch("gemv", f"nk_gemv_out_{ctag}{sw}", (-(-plane // 64), 1, 1), (256, 1, 1), out,
-                           bytes=4 * ks * plane * len(launches) + plane * c_dtype.itemsize))
+    launches.append(_reduce_planes(out, c_dtype, swiglu))
     return launches
+
+
+def _reduce_planes(args: "GemvArgs", c_dtype, swiglu: bool) -> Launch:
+    """The launch that adds a projection's partial planes and applies the
+    epilogue: one wave per four ranges over 64 outputs, or, from
+    ``REDUCE4_MIN`` outputs on, four outputs per thread (24 x 4096 from 8
+    planes 4.8 us either way, 64 x 6144 from 5 planes 9.1 against 5.0)."""
+    out = GemvArgs.from_buffer_copy(args)
+    plane = out.M * out.N
+    vb = 4 * c_dtype.itemsize
+    four = (plane >= REDUCE4_MIN and out.N % 4 == 0 and out.ldc % 4 == 0 and out.C % vb == 0
+            and (not out.resid or out.resid % vb == 0))
+    if four:
+        out.flags |= GEMV_OUT4
+    ctag = "bf16" if c_dtype == dt.bfloat16 else "f32"
+    return Launch("gemv", f"nk_gemv_out_{ctag}" + ("_swiglu" if swiglu else ""),
+                  (-(-plane // (1024 if four else 64)), 1, 1), (256, 1, 1), out,
+                  bytes=4 * out.ksplit * plane * (2 if swiglu else 1) + plane * c_dtype.itemsize)
 
 
 # ---------------------------------------------------------------------------
@@ -604,12 +686,10 @@ def gemv(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
     btag = "e4m3" if fp8 else "bf16"
     sw = "_swiglu" if swiglu else ""
     n_mm = 2 if swiglu else 1
-    ctag = "bf16" if c_dtype == dt.bfloat16 else "f32"
     return [Launch("gemv", f"nk_gemv_{layout}_{btag}{sw}_m{mt}", (blocks * ks, 1, 1), (256, 1, 1), args,
                    bytes=M * K * 2 + n_mm * N * K * b_dtype.itemsize + 4 * ks * M * N * n_mm,
                    flops=2 * M * N * K * n_mm),
-            Launch("gemv", f"nk_gemv_out_{ctag}{sw}", (-(-M * N // 64), 1, 1), (256, 1, 1), args,
-                   bytes=4 * ks * M * N * n_mm + M * N * c_dtype.itemsize)]
+            _reduce_planes(args, c_dtype, swiglu)]
 
 
 GEMV_MFMA_MAX_M = 32
@@ -716,13 +796,11 @@ def gemv_mfma(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, c_d
     n_mm = 2 if swiglu else 1
     sw = "_swiglu" if swiglu else ""
     btag = "e4m3" if fp8 else "bf16"
-    ctag = "bf16" if c_dtype == dt.bfloat16 else "f32"
     blocks = -(-N // (128 if swiglu else 256))
     return [Launch("gemv", f"nk_gemv_mfma_{layout}_{btag}{sw}_t{tiles}", (blocks * ks, 1, 1), (256, 1, 1), args,
                    bytes=M * K * 2 + n_mm * N * K * b_dtype.itemsize + 4 * ks * M * N * n_mm,
                    flops=2 * M * N * K * n_mm),
-            Launch("gemv", f"nk_gemv_out_{ctag}{sw}", (-(-M * N // 64), 1, 1), (256, 1, 1), args,
-                   bytes=4 * ks * M * N * n_mm + M * N * c_dtype.itemsize)]
+            _reduce_planes(args, c_dtype, swiglu)]
 
 
 class HeadRopeTarget(ctypes.Structure):

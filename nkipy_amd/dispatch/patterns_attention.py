@@ -585,13 +585,15 @@ class QkvRopeMatch(Match):
         Hk = rk.roles[0][2]
         hd = LA.GemmRope.HEAD_DIM
         cos, sin = rq.cos, rq.sin
+        # (the tile of the plain projection in one K loop: the same sums)
+        tile = LA.gemm_form(M, N, K, w.layout, w.value.dtype == dt.float8_e4m3fn, ranges=False)[0]
 
         def make(addr):
             rope = LA.GemmRope(addr(cos.base) + 4 * cos.offset, addr(sin.base) + 4 * sin.offset,
                                addr(rq.out), addr(rk.out), t_ss, S, Hq * hd, Hk * hd)
             return LA.gemm(addr(x), addr(w.value), addr(out), M, N, K, layout=w.layout,
                            b_dtype=w.value.dtype, c_dtype=out.dtype, ldb=ldb,
-                           scale_ptr=addr(w.scale) if w.scale is not None else 0, rope=rope)
+                           scale_ptr=addr(w.scale) if w.scale is not None else 0, rope=rope, tile=tile)
 
         desc = (f"gemm {w.layout} M={M} N={N} K={K} {dt.name(w.value.dtype)} -> bf16 "
                 f"+rope q {Hq}x{hd} k {Hk}x{hd}")

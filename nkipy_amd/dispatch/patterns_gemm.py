@@ -173,9 +173,7 @@ class GemmMatch(Match):
         rnd_bias, rnd_resid = self.rnd
 
         # a few rows (a decode token per sequence): the split-K projection,
-        # which streams the weights over the whole part; up to a tile of rows
-        # (a decode batch): the MFMA kernels over K ranges, so that the
-        # grid fills the part
+        # which streams the weights over the whole part
         fp8 = w.value.dtype == dt.float8_e4m3fn
         # a projection of up to 16-32 rows: the MFMA form of the few-row
         # kernels (16-row tiles, weights streamed once)
@@ -183,8 +181,10 @@ class GemmMatch(Match):
                 and (up is None or (up.layout == w.layout and up.value.dtype == w.value.dtype))
                 and LA.gemv_mfma_preferred(M, N, K, up is not None, w.layout, fp8))
         small = not mfma and LA.gemv_preferred(M, w.layout, fp8)
-        splitk = (self.split_k and not mfma and not small and not (fp8 and w.layout == "nn")
-                  and LA.gemm_splitk_useful(M, N, K, up is not None, fp8))
+        # any more rows: output tiles of 256 or 128, over K ranges where the
+        # tiles leave CUs idle
+        tile, ks_g, kc_g = LA.gemm_form(M, N, K, w.layout, fp8, up is not None, self.split_k)
+        splitk = not mfma and not small and ks_g > 1
         small = small or (not mfma and M <= LA.GEMV_MAX_M and not splitk)
         ws = None
         fold = False
@@ -198,8 +198,7 @@ class GemmMatch(Match):
             ws = Slot(plan.add_buffer(LA.gemv_workspace_bytes(M, N, K, w.layout, fp8, up is not None), "temp",
                                       "gemv.partials"))
         elif splitk:
-            ws = Slot(plan.add_buffer(LA.gemm_splitk_workspace_bytes(M, N, K, up is not None, fp8), "temp",
-                                      "gemm.partials"))
+            ws = Slot(plan.add_buffer(4 * ks_g * M * N * (2 if up is not None else 1), "temp", "gemm.partials"))
 
         def make(addr):
             up_ptr = 0
@@ -232,14 +231,15 @@ class GemmMatch(Match):
                                       scale_ptr=addr(w.scale) if w.scale is not None else 0,
                                       resid_ptr=addr(resid) if resid is not None else 0,
                                       up_ptr=up_ptr, up_scale_ptr=up_scale,
-                                      round_before_bias=rnd_bias, round_before_resid=rnd_resid)
+                                      round_before_bias=rnd_bias, round_before_resid=rnd_resid,
+                                      split=(ks_g, kc_g))
             return LA.gemm(addr(x), addr(w.value), addr(out), M, N, K, layout=w.layout,
                            b_dtype=w.value.dtype, c_dtype=out.dtype, ldb=ldb,
                            bias_ptr=addr(bias) if bias is not None else 0,
                            scale_ptr=addr(w.scale) if w.scale is not None else 0,
                            resid_ptr=addr(resid) if resid is not None else 0,
                            up_ptr=up_ptr, up_scale_ptr=up_scale,
-                           round_before_bias=rnd_bias, round_before_resid=rnd_resid)
+                           round_before_bias=rnd_bias, round_before_resid=rnd_resid, tile=tile)
 
         kind = "gemm_swiglu" if up is not None else "gemm"
         desc = (f"{'swiglu ' if up is not None else ''}gemm {w.layout} M={M} N={N} K={K} "
