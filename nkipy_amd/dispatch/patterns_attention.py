@@ -222,7 +222,7 @@ class HeadRopeMatch(Match):
                 # the rows, or their fp32 partial sums at the same element offset
                 x_ptr = addr(planes[0]) + 4 * xv.offset if planes else addr(xv.base) + 2 * xv.offset
                 specs.append(LA.HeadRopeSpec(
-                    x_ptr, addr(m["out"]), m["H"], m["x_str"], m["o_str"], m["x_half"],
+                    x_ptr, addr(m["out"]) + 2 * m.get("o_off", 0), m["H"], m["x_str"], m["o_str"], m["x_half"],
                     norm=nm is not None, eps=nm.eps if nm is not None else 0.0,
                     w_ptr=addr(nm.w) if nm is not None and nm.w is not None else 0,
                     mul_recip=bool(nm.mul_recip) if nm is not None else False,
@@ -236,7 +236,8 @@ class HeadRopeMatch(Match):
 
         parts = [(f"copy {m['H']} heads" if m.get("copy") else
                   f"{'rmsnorm + ' if m['norm'] is not None else ''}rope {m['H']} heads")
-                 + (" -> cache row" if m.get("o_pos") else "") for m in members]
+                 + (" -> cache row" if m.get("o_pos") else "") + ("s" if m.get("o_pos") == (0, 0) else "")
+                 for m in members]
         desc = f"head rope B={B} S={S} D={D} bf16 steps: " + ", ".join(parts) + \
             (" (runtime position)" if tb["pos"] is not None else "") + \
             (f" from {planes[1]} partial-sum planes" if planes else "")
@@ -473,43 +474,73 @@ class HeadRopePattern:
         A = P.shape[1]
         return {"node": node, "src": src, "out": node.out, "o_str": (A * H * D, 0, D), "o_pos": (H * D, A)}
 
-    def _cache_writes(self, L, ms, tb):
-        """The decode form (one token, tables taken at the runtime position,
-        q and a normalised k of one projection): k written into its cache
-        row by the launch instead of by a scatter step, and the v heads of
-        the same projection copied into theirs (a third target).  Returns
-        the members with those writes, or None."""
-        if len(ms) != 2 or tb["pos"] is None or ms[0]["bsd"][1] != 1:
+    @staticmethod
+    def _update(L, node, B, S, H, D):
+        """``cache[:, s0:s0 + S] = src`` (attention.py:101-105 without
+        start_pos) as an in-place update of a cache argument the kernel's
+        output aliases; the fields of :meth:`_scatter`, the rows at a fixed
+        offset."""
+        if node.op != "dynamic_update_slice" or id(node) in L.covered:
             return None
-        B, _, D = ms[0]["bsd"]
+        P, src = node.inputs
+        st = [int(v) for v in node.attrs["start"]]
+        if not P.is_parameter or P.dtype != dt.bfloat16 or P.ndim != 4 or P.shape[0] != B or \
+                tuple(P.shape[2:]) != (H, D) or tuple(src.shape) != (B, S, H, D) or src.dtype != dt.bfloat16:
+            return None
+        if (st[0], st[2], st[3]) != (0, 0, 0) or not 0 <= st[1] <= P.shape[1] - S:
+            return None
+        if len(L.users.get(P.id, [])) != 1:  # nothing else reads the cache before its update
+            return None
+        if not any(L.g.results[a.output_index] is node.out and f"{a.param_name}.must_alias_input" == P.name
+                   for a in L.g.aliases):
+            return None
+        A = P.shape[1]
+        return {"node": node, "src": src, "out": node.out, "o_str": (A * H * D, H * D, D), "o_pos": (0, 0),
+                "o_off": st[1] * H * D}
+
+    def _cache_writes(self, L, ms, tb):
+        """The caches written by the launch instead of by scatter / update
+        steps: q and a normalised k of one projection, k into its cache rows
+        and the v heads of the same projection copied into theirs (a third
+        target).  One token at the runtime position (decode) or S tokens at a
+        fixed one (prefill: 1500 tokens of 32 / 8 heads, the v slice and the
+        two update steps 113 us, 1.4 us more of this launch).  Returns
+        the members with those writes, or None."""
+        if len(ms) != 2 or (tb["pos"] is not None and ms[0]["bsd"][1] != 1):
+            return None
+        B, S, D = ms[0]["bsd"]
         pos = tb["pos"]
+        if pos is not None:
+            op, write = "scatter_along_axis", lambda n, H: self._scatter(L, n, pos, B, H, D)
+        else:
+            op, write = "dynamic_update_slice", lambda n, H: self._update(L, n, B, S, H, D)
         kk = [i for i, m in enumerate(ms) if m["norm"] is not None and m["out"].id not in L.result_ids
               and len(L.users.get(m["out"].id, [])) == 1]
         for i in kk:
             km = ms[i]
-            kw = self._scatter(L, L.users[km["out"].id][0], pos, B, km["H"], D)
+            kw = write(L.users[km["out"].id][0], km["H"])
             if kw is None or kw["src"] is not km["out"]:
                 continue
             base = km["x"].base
             for n in L.live:
-                if n is kw["node"] or n.op != "scatter_along_axis":
+                if n is kw["node"] or n.op != op:
                     continue
-                src = n.inputs[2]
+                src = n.inputs[-1]
                 vv = resolve(src, widen_ok=False)
                 if vv.base is not base or src.ndim != 4:
                     continue
-                vw = self._scatter(L, n, pos, B, src.shape[2], D)
+                vw = write(n, src.shape[2])
                 if vw is None:
                     continue
                 st = [vv.simple(d) for d in range(4)]
                 if any(v is None for v in st) or st[3] != 1:
                     continue
                 out = [dict(m) for m in ms]
-                out[i].update(out=kw["out"], o_str=kw["o_str"], o_pos=kw["o_pos"],
+                out[i].update(out=kw["out"], o_str=kw["o_str"], o_pos=kw["o_pos"], o_off=kw.get("o_off", 0),
                               nodes=km["nodes"] + [kw["node"]])
                 out.append({"n": n, "nodes": [n], "chain": list(vv.nodes), "x": vv, "x_str": tuple(st[:3]),
                             "x_half": D // 2, "H": src.shape[2], "out": vw["out"], "o_str": vw["o_str"],
-                            "o_pos": vw["o_pos"], "norm": None, "copy": True, "bsd": km["bsd"]})
+                            "o_pos": vw["o_pos"], "o_off": vw.get("o_off", 0), "norm": None, "copy": True, "bsd": km["bsd"]})
                 return out
         return None
 

@@ -264,3 +264,45 @@ def test_head_rope_adds_projection_planes(gpu, B, H, Hkv, D, hid, planes):
     for k in outs[0]:
         np.testing.assert_array_equal(outs[0][k], outs[1][k], err_msg=k)
     assert not np.signbit(dt.to_float32(outs[0]["cache_v"])[0, pos]).any()
+
+
+def _prefill_with_cache(H, Hkv, D, start):
+    def fn(qkv, q_norm_weight, k_norm_weight, cache_k, cache_v):
+        B, S, _ = qkv.shape
+        xq, xk, xv = np.split(qkv, [H * D, (H + Hkv) * D], axis=2)
+        xq = rmsnorm_kernel(xq.reshape(B, S, H, D), q_norm_weight, EPS)
+        xk = rmsnorm_kernel(xk.reshape(B, S, Hkv, D), k_norm_weight, EPS)
+        cos, sin = compute_cos_sin_cache(D, cache_k.shape[1], base=THETA)
+        cos = tensor_apis.constant(cos).astype(qkv.dtype)[start:start + S]
+        sin = tensor_apis.constant(sin).astype(qkv.dtype)[start:start + S]
+        xq, xk = apply_rotary_emb_kernel(xq, xk, cos, sin)
+        cache_k[:, start:start + S] = xk
+        cache_v[:, start:start + S] = xv.reshape(B, S, Hkv, D)
+        return xq
+    return fn
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,D,maxs,start", [(1, 5, 4, 2, 128, 16, 0), (2, 33, 8, 2, 64, 64, 0),
+                                                     (3, 100, 4, 4, 128, 256, 7), (1, 31, 2, 1, 128, 32, 1)])
+def test_prefill_prologue_writes_the_caches(gpu, B, S, H, Hkv, D, maxs, start):
+    """S tokens at a fixed offset: k and v go into their cache rows by the
+    prologue's launch; q, the written rows and the rows around them equal the
+    generic lowering's bit for bit."""
+    print(f"prefill prologue B={B} S={S} H={H}/{Hkv} D={D} start={start}", flush=True)
+    rng = np.random.default_rng(S + H)
+    arrays = [rng.standard_normal((B, S, (H + 2 * Hkv) * D)), rng.uniform(0.5, 1.5, D), rng.uniform(0.5, 1.5, D),
+              rng.standard_normal((B, maxs, Hkv, D)), rng.standard_normal((B, maxs, Hkv, D))]
+    args = [dt.to_bf16(N.bf16_round(a)) for a in arrays]
+    g = NKIPyKernel.trace(_prefill_with_cache(H, Hkv, D, start)).specialize(*args)
+    fused = lower(g)
+    generic = lower(g, [p for p in default_patterns() if not isinstance(p, HeadRopePattern)])
+    assert fused.kernel_kinds == ["head_rope"], fused.kernel_kinds
+    names = [p.name for p in g.parameters]
+    outs = []
+    for i, plan in enumerate((fused, generic)):
+        dk = DeviceKernel(g, plan, f"prefill_prologue_{i}")
+        res = dk({n: DeviceTensor.from_numpy(a, name=n) for n, a in zip(names, args)})
+        outs.append({k: dt.numpy_storage(v.numpy()) for k, v in res.items()})
+    assert set(outs[0]) == set(outs[1]) and len(outs[0]) == 3
+    for k in outs[0]:
+        np.testing.assert_array_equal(outs[0][k], outs[1][k], err_msg=k)
