@@ -547,3 +547,98 @@ extern "C" __global__ __launch_bounds__(256) void nk_topk(TopkArgs a) {
     __syncthreads();
   }
 }
+
+// Row-wise top-k of long rows, in two launches (nk_topk walks a row with one
+// workgroup: 250 us for 8 rows of 151936, one memory round trip per 256
+// elements; 5.4 + 4.0 us in this form, launches mostly).  A segment of TK_SEG elements is held in registers by one
+// workgroup, which picks its k best; one workgroup per row then picks the k
+// best of the segments' picks.  Elements are compared as 64-bit keys: the
+// value mapped to an unsigned order (largest first; -0 as +0) above the
+// complement of the index, so a larger key is a larger value or, among equals,
+// a smaller index, and no two are equal: the picks and their order are those
+// of nk_topk.  A NaN's key is 0, which no pick takes before any number, as
+// there.  fp32, fp16 and bf16 rows.
+#define TK_PER 16
+#define TK_SEG (256 * TK_PER)
+struct TopkSegArgs {
+  const void *in;
+  uint64_t *keys;  // rows x nseg x k
+  uint32_t *idx;   // rows x k
+  int64_t n;
+  int32_t nseg, k, largest, dtype;
+};
+
+__device__ __forceinline__ uint64_t topk_key(float v, float sgn, uint32_t i) {
+  const float x = sgn * v + 0.f;
+  const uint32_t u = __float_as_uint(x);
+  const uint32_t o = (u & 0x80000000u) ? ~u : u | 0x80000000u;
+  return x != x ? 0 : ((uint64_t)o << 32) | (uint32_t)~i;
+}
+// the workgroup's largest key (all 256 threads get it)
+__device__ __forceinline__ uint64_t topk_max(uint64_t m, uint64_t *sv) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t x = __shfl_xor((unsigned long long)m, o, 64);
+    m = x > m ? x : m;
+  }
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sv[threadIdx.x >> 6] = m;
+  __syncthreads();
+  const uint64_t a = sv[0] > sv[1] ? sv[0] : sv[1], b = sv[2] > sv[3] ? sv[2] : sv[3];
+  return a > b ? a : b;
+}
+
+extern "C" __global__ __launch_bounds__(256) void nk_topk_segments(TopkSegArgs a) {
+  __shared__ uint64_t sv[4];
+  const int64_t row = blockIdx.x / (uint32_t)a.nseg;
+  const int seg = blockIdx.x % (uint32_t)a.nseg;
+  const int64_t base = row * a.n;
+  const float sgn = a.largest ? 1.f : -1.f;
+  const int esz = a.dtype == DT_F32 ? 4 : 2;
+  const uint8_t *p = (const uint8_t *)a.in + base * esz;
+  const bool vec = ((uintptr_t)p & 15) == 0;
+  uint64_t key[TK_PER];
+  // thread t: elements 8 t .. 8 t + 7 of each half of the segment
+#pragma unroll
+  for (int h = 0; h < TK_PER / 8; ++h) {
+    const int64_t j0 = (int64_t)seg * TK_SEG + h * 2048 + threadIdx.x * 8;
+    float v[8];
+    if (vec && j0 + 8 <= a.n) {
+      if (a.dtype == DT_F32) Vec8<float>::load((const float *)p + j0, v);
+      else if (a.dtype == DT_BF16) Vec8<bf16>::load((const bf16 *)p + j0, v);
+      else Vec8<f16>::load((const f16 *)p + j0, v);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = j0 + e < a.n ? (float)load_any(p, j0 + e, a.dtype) : __builtin_nanf("");
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) key[h * 8 + e] = topk_key(v[e], sgn, (uint32_t)(j0 + e));
+  }
+  uint64_t prev = ~0ull;
+  uint64_t *out = a.keys + (int64_t)blockIdx.x * a.k;
+  for (int r = 0; r < a.k; ++r) {
+    uint64_t m = 0;
+#pragma unroll
+    for (int e = 0; e < TK_PER; ++e) m = key[e] < prev && key[e] > m ? key[e] : m;
+    prev = topk_max(m, sv);
+    if (threadIdx.x == 0) out[r] = prev;
+  }
+}
+
+extern "C" __global__ __launch_bounds__(256) void nk_topk_merge(TopkSegArgs a) {
+  __shared__ uint64_t sv[4];
+  const int64_t row = blockIdx.x;
+  const int cnt = a.nseg * a.k;
+  const uint64_t *in = a.keys + row * cnt;
+  uint64_t prev = ~0ull;
+  for (int r = 0; r < a.k; ++r) {
+    uint64_t m = 0;
+    for (int j = threadIdx.x; j < cnt; j += 256) {
+      const uint64_t x = in[j];
+      m = x < prev && x > m ? x : m;
+    }
+    prev = topk_max(m, sv);
+    // nothing left but NaN: the last element, as nk_topk
+    if (threadIdx.x == 0) a.idx[row * a.k + r] = prev ? (uint32_t)~(uint32_t)prev : (uint32_t)(a.n - 1);
+  }
+}

@@ -20,7 +20,7 @@ import numpy as np
 from nkipy_amd.core import dtypes as dt
 from nkipy_amd.core.backend.ir import Value
 from nkipy_amd.dispatch.launchers import Launch, LaunchError
-from nkipy_amd.dispatch.plan import Step
+from nkipy_amd.dispatch.plan import Slot, Step
 
 # ---------------------------------------------------------------------------
 # dtype codes and op codes shared with csrc/kernels/generic.hip
@@ -588,18 +588,37 @@ class TopkArgs(ctypes.Structure):
                 ("dtype", ctypes.c_int32), ("pad", ctypes.c_int32)]
 
 
+class TopkSegArgs(ctypes.Structure):
+    _fields_ = [("inp", ctypes.c_void_p), ("keys", ctypes.c_void_p), ("idx", ctypes.c_void_p),
+                ("n", ctypes.c_int64), ("nseg", ctypes.c_int32), ("k", ctypes.c_int32),
+                ("largest", ctypes.c_int32), ("dtype", ctypes.c_int32)]
+
+
+TOPK_SEG = 4096        # elements per workgroup of the segment form
+TOPK_SEG_MIN = 8192    # row length from which the segment form is taken
+TOPK_SEG_MAX_K = 16
+
+
 class TopkStep(Step):
     """Indices of the k largest (or smallest) elements of each row along the
-    last axis, ordered by value, ties by index (nk_topk)."""
+    last axis, ordered by value, ties by index (nk_topk).  Rows of two
+    segments and more of a float type take the segment form, up to 16 picks
+    (each costs every workgroup a reduction): 8 rows of 151936 bf16, one
+    pick, 5.4 + 4.0 us against 250."""
 
     kind = "topk"
 
-    def __init__(self, node):
+    def __init__(self, node, plan=None):
         x = node.inputs[0]
         super().__init__("topk", [x], [node.out])
         self.node, self.x = node, x
         self.n = x.shape[-1] if x.ndim else 1
         self.rows = x.size // max(self.n, 1)
+        self.nseg, self.keys = -(-self.n // TOPK_SEG), None
+        k = int(node.attrs["k"])
+        if (plan is not None and TOPK_SEG_MIN <= self.n < 2**32 and 0 < k <= TOPK_SEG_MAX_K and self.rows > 0
+                and x.dtype in (dt.float32, dt.float16, dt.bfloat16) and self.rows * self.nseg < 2**31):
+            self.keys = Slot(plan.add_buffer(8 * self.rows * self.nseg * k, "temp", "topk.keys"))
 
     def launches(self, addr):
         at = self.node.attrs
@@ -607,6 +626,14 @@ class TopkStep(Step):
             return []
         if self.rows >= 2**31:
             raise LaunchError("topk: too many rows")
+        if self.keys is not None:
+            k = int(at["k"])
+            a = TopkSegArgs(addr(self.x), addr(self.keys), addr(self.node.out), self.n, self.nseg, k,
+                            1 if at["largest"] else 0, dtype_code(self.x.dtype))
+            return [Launch("generic", "nk_topk_segments", (self.rows * self.nseg, 1, 1), (256, 1, 1), a,
+                           bytes=self.rows * self.n * self.x.dtype.itemsize),
+                    Launch("generic", "nk_topk_merge", (self.rows, 1, 1), (256, 1, 1), a,
+                           bytes=8 * self.rows * self.nseg * k)]
         a = TopkArgs(addr(self.x), addr(self.node.out), self.rows, self.n, int(at["k"]),
                      1 if at["largest"] else 0, dtype_code(self.x.dtype), 0)
         return [Launch("generic", "nk_topk", (self.rows, 1, 1), (256, 1, 1), a,

@@ -336,7 +336,7 @@ class Lowering:
         if op == "cumsum":
             return [G.CumsumStep(n)]
         if op == "topk":
-            return [G.TopkStep(n)]
+            return [G.TopkStep(n, plan)]
         if op == "concatenate":
             ax = n.attrs["dimension"]
             s = G.contiguous_strides(v.shape)

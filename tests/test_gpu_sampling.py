@@ -63,3 +63,31 @@ def test_greedy_sampling(gpu):
     # the pick is a largest bf16 logit (ties between equal bf16 logits would
     # be a legitimate difference; none occur at this seed)
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("d", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("rows,n,k", [(1, 8192, 1), (3, 8193, 3), (2, 12289, 16), (5, 40000, 2)])
+@pytest.mark.parametrize("asc", [False, True])
+def test_topk_of_long_rows(gpu, rows, n, k, asc, d):
+    """The segment form: ties (few distinct values, both zeros), infinities
+    and partial last segments, against a stable sort."""
+    print(f"topk segments {rows}x{n} k={k} asc={asc} {d}", flush=True)
+    rng = np.random.default_rng(n + k)
+    x = rng.integers(-40, 41, (rows, n)).astype(np.float32) * 0.25
+    x[rng.random((rows, n)) < 0.01] = -0.0
+    x[:, ::1777] = np.float32(np.inf)
+    x[:, 5::1999] = np.float32(-np.inf)
+    x[0, :] = np.float32(-np.inf) if not asc else np.float32(np.inf)  # every element equal, at the worst value
+    xs = dt.to_bf16(x) if d == "bfloat16" else x.astype(d)
+    _, i = baremetal_jit(_topk_kernel(k, asc))(xs)
+    ref = np.argsort(x if asc else -x, axis=-1, kind="stable")[:, :k]
+    np.testing.assert_array_equal(i, ref)
+
+
+def test_topk_segments_past_nan(gpu):
+    """Rows with NaN: no pick takes one while numbers are left, as the
+    one-workgroup form."""
+    x = np.full((2, 9000), np.nan, np.float32)
+    x[0, [17, 8999]] = [1.0, 2.0]
+    _, i = baremetal_jit(_topk_kernel(2, False))(x)
+    np.testing.assert_array_equal(i, [[8999, 17], [8999, 8999]])
