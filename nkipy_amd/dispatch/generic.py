@@ -19,7 +19,7 @@ import numpy as np
 
 from nkipy_amd.core import dtypes as dt
 from nkipy_amd.core.backend.ir import Value
-from nkipy_amd.dispatch.launchers import Launch, LaunchError
+from nkipy_amd.dispatch.launchers import GemvArgs, Launch, LaunchError, _reduce_planes
 from nkipy_amd.dispatch.plan import Slot, Step
 
 # ---------------------------------------------------------------------------
@@ -476,12 +476,67 @@ class ReduceStep(Step):
         return [Launch("generic", "nk_reduce", (n_out, 1, 1), (256, 1, 1), a)]
 
 
+class DotF32Args(ctypes.Structure):
+    _fields_ = [
+        ("A", ctypes.c_void_p), ("B", ctypes.c_void_p), ("C", ctypes.c_void_p),
+        ("batch", ctypes.c_int64), ("M", ctypes.c_int64), ("N", ctypes.c_int64), ("K", ctypes.c_int64),
+        ("sab", ctypes.c_int64), ("sam", ctypes.c_int64), ("sak", ctypes.c_int64),
+        ("sbb", ctypes.c_int64), ("sbk", ctypes.c_int64), ("sbn", ctypes.c_int64),
+        ("a_dtype", ctypes.c_int32), ("b_dtype", ctypes.c_int32), ("c_dtype", ctypes.c_int32),
+        ("a_mode", ctypes.c_int32), ("b_mode", ctypes.c_int32), ("ksplit", ctypes.c_int32),
+        ("kc", ctypes.c_int32), ("c_vec", ctypes.c_int32),
+        ("a_bytes", ctypes.c_int32), ("b_bytes", ctypes.c_int32),
+    ]
+
+
+_DOT_F32 = {dt.float32: 0, dt.float16: 1, dt.bfloat16: 2}
+DOT_TILE = 64
+DOT_TARGET_WGS = 768  # three workgroups per CU
+DOT_MIN_RANGE = 128   # k per range
+
+
+def dot_split(batch: int, M: int, N: int, K: int) -> Tuple[int, int]:
+    """(ranges, k per range) of :class:`DotStep`'s matrix-core form: K ranges
+    when the tiles alone do not give every CU three workgroups (us, one range
+    / as many as do: 200 x 1024 x 3072 101 / 24, 200 x 6144 x 1024 45 / 38, 1
+    x 2048 x 8192 276 / 24; 1024 x 3072 x 1024, 768 tiles, 59 in one, 66 in
+    two), of 128 k at least."""
+    tiles = batch * -(-M // DOT_TILE) * -(-N // DOT_TILE)
+    ks = max(1, min(DOT_TARGET_WGS // tiles, K // DOT_MIN_RANGE, 65535 // batch))
+    while ks > 1 and 4 * ks * batch * M * N > 1 << 27:
+        ks -= 1
+    kc = -(-(-(-K // ks)) // 32) * 32 if K else 32
+    return max(1, -(-K // kc)), kc
+
+
+def _dot_mode(ptr: int, esz: int, s_row: int, s_k: int, s_batch: int, rows: int, K: int, batch: int) -> int:
+    """Load mode of an operand: four elements at a time along k (1) or along
+    its rows / columns (2) when they are contiguous and every such piece is
+    whole and aligned, else one (0)."""
+    if ptr % (4 * esz) or (batch > 1 and s_batch % 4):
+        return 0
+    if s_k == 1 and K % 4 == 0 and (s_row % 4 == 0 or rows == 1):
+        return 1
+    return 2 if s_row == 1 and rows % 4 == 0 and s_k % 4 == 0 else 0
+
+
+def _dot_span(esz: int, s_row: int, s_k: int, rows: int, K: int) -> int:
+    """Bytes from an operand's first element to the end of its last (one
+    batch); negative strides, which a buffer resource cannot address, give
+    no span."""
+    if s_row < 0 or s_k < 0:
+        return 1 << 62
+    return ((max(rows, 1) - 1) * s_row + (max(K, 1) - 1) * s_k + 1) * esz
+
+
 class DotStep(Step):
-    """Fallback batched dot with arbitrary operand strides (fp32 accumulate)."""
+    """Fallback batched dot with arbitrary operand strides (fp32 accumulate):
+    fp32, fp16 and bf16 operands on the matrix cores (nk_dot_f32), other
+    types on nk_dot."""
 
     kind = "dot"
 
-    def __init__(self, node, lhs, rhs):
+    def __init__(self, node, lhs, rhs, plan=None):
         super().__init__("dot (generic)", [lhs[0], rhs[0]], [node.out])
         self.node = node
         a_v, a_s, a_o = lhs
@@ -517,8 +572,56 @@ class DotStep(Step):
         self.sbn = int(b_s[rf[0]]) if rf else 0
         self.sbk = int(b_s[rc[0]])
         self.a_v, self.a_o, self.b_v, self.b_o = a_v, a_o, b_v, b_o
+        # (operands are addressed with 32-bit offsets, whole stages past their end)
+        span = max(_dot_span(a_v.dtype.itemsize, self.sam, self.sak, self.M + DOT_TILE, self.K + 2 * DOT_TILE),
+                   _dot_span(b_v.dtype.itemsize, self.sbn, self.sbk, self.N + DOT_TILE, self.K + 2 * DOT_TILE))
+        self.f32 = all(v.dtype in _DOT_F32 for v in (a_v, b_v, node.out)) and span < 2**31
+        self.split, self.planes = (1, self.K), None
+        outputs = self.batch * self.M * self.N
+        if self.f32 and plan is not None and outputs > 0:
+            # (the reduction writes fp32 or bf16)
+            ks, kc = dot_split(self.batch, self.M, self.N, self.K)
+            if ks > 1 and node.out.dtype != dt.float16 and outputs < 2**31:
+                self.split = ks, kc
+                self.planes = Slot(plan.add_buffer(4 * ks * outputs, "temp", "dot.partials"))
+
+    def _launches_f32(self, addr):
+        ks, kc = self.split
+        a = DotF32Args()
+        a.A = addr(self.a_v) + self.a_o * self.a_v.dtype.itemsize
+        a.B = addr(self.b_v) + self.b_o * self.b_v.dtype.itemsize
+        out, ctype = addr(self.node.out), self.node.out.dtype
+        a.C = addr(self.planes) if ks > 1 else out
+        a.batch, a.M, a.N, a.K = self.batch, self.M, self.N, self.K
+        a.sab, a.sam, a.sak = self.sab, self.sam, self.sak
+        a.sbb, a.sbk, a.sbn = self.sbb, self.sbk, self.sbn
+        a.a_dtype, a.b_dtype = _DOT_F32[self.a_v.dtype], _DOT_F32[self.b_v.dtype]
+        a.c_dtype = 0 if ks > 1 else _DOT_F32[ctype]
+        esa, esb = self.a_v.dtype.itemsize, self.b_v.dtype.itemsize
+        a.a_mode = _dot_mode(a.A, esa, self.sam, self.sak, self.sab, self.M, self.K, self.batch)
+        a.b_mode = _dot_mode(a.B, esb, self.sbn, self.sbk, self.sbb, self.N, self.K, self.batch)
+        a.a_bytes = _dot_span(esa, self.sam, self.sak, self.M, self.K)
+        a.b_bytes = _dot_span(esb, self.sbn, self.sbk, self.N, self.K)
+        a.ksplit, a.kc = ks, kc if ks > 1 else -(-max(self.K, 1) // 32) * 32
+        a.c_vec = 1 if a.c_dtype == 0 and self.N % 4 == 0 and a.C % 16 == 0 else 0
+        rows = self.batch * self.M
+        sym = f"nk_dot_f32_{'f' if esa == 4 else 'h'}{a.a_mode}_{'f' if esb == 4 else 'h'}{a.b_mode}"
+        ls = [Launch("dotf32", sym, (-(-self.N // DOT_TILE), -(-self.M // DOT_TILE), self.batch * ks),
+                     (256, 1, 1), a, flops=2 * rows * self.N * self.K)]
+        if ks > 1:
+            red = GemvArgs(None, None, None, out, None, None, None, None, a.C, rows, self.N, self.K, self.K, self.K,
+                           self.N, ks, kc, 0, 0)
+            ls.append(_reduce_planes(red, ctype, False))
+        return ls
 
     def launches(self, addr):
+        if self.M * self.N * self.batch == 0:
+            return []
+        gx, gy = (self.N + 15) // 16, (self.M + 15) // 16
+        if gy > 65535 or self.batch > 65535:
+            raise LaunchError("generic dot grid too large")
+        if self.f32:
+            return self._launches_f32(addr)
         a = DotArgs()
         a.A = addr(self.a_v) + self.a_o * self.a_v.dtype.itemsize
         a.B = addr(self.b_v) + self.b_o * self.b_v.dtype.itemsize
@@ -529,11 +632,6 @@ class DotStep(Step):
         a.a_dtype = dtype_code(self.a_v.dtype)
         a.b_dtype = dtype_code(self.b_v.dtype)
         a.c_dtype = dtype_code(self.node.out.dtype)
-        gx, gy = (self.N + 15) // 16, (self.M + 15) // 16
-        if self.M * self.N * self.batch == 0:
-            return []
-        if gy > 65535 or self.batch > 65535:
-            raise LaunchError("generic dot grid too large")
         return [Launch("generic", "nk_dot", (gx, gy, self.batch), (256, 1, 1), a,
                        flops=2 * self.batch * self.M * self.N * self.K)]
 

@@ -327,7 +327,7 @@ class Lowering:
             else:
                 lhs = G.strided_access(n.inputs[0], self.is_mat)
                 rhs = G.strided_access(n.inputs[1], self.is_mat)
-            return [G.DotStep(n, lhs, rhs)]
+            return [G.DotStep(n, lhs, rhs, plan)]
         if op in ("take", "take_along_axis"):
             return [G.GatherStep(n)]
         if op in ("scatter_along_axis", "put_along_axis"):
