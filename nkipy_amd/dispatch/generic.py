@@ -96,6 +96,50 @@ class EwArgs(ctypes.Structure):
     ]
 
 
+class EwfInput(ctypes.Structure):
+    _fields_ = [("ptr", ctypes.c_void_p), ("strides", ctypes.c_int32 * EW_MAX_RANK),
+                ("dtype", ctypes.c_int32), ("mode", ctypes.c_int32)]
+
+
+class EwfInstr(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_uint8) for n in ("op", "dst", "a", "b", "c", "dtype")] + \
+        [("pad", ctypes.c_uint8 * 2), ("imm", ctypes.c_float)]
+
+
+class EwfArgs(ctypes.Structure):
+    _fields_ = [
+        ("out", ctypes.c_void_p), ("out_strides", ctypes.c_int32 * EW_MAX_RANK),
+        ("shape", ctypes.c_uint32 * EW_MAX_RANK), ("total", ctypes.c_uint32), ("step", ctypes.c_uint32),
+        ("rank", ctypes.c_int32), ("n_instr", ctypes.c_int32), ("out_dtype", ctypes.c_int32),
+        ("out_mode", ctypes.c_int32), ("result_reg", ctypes.c_int32), ("rows4", ctypes.c_int32),
+        ("inp", EwfInput * EW_MAX_IN), ("prog", EwfInstr * EW_MAX_INSTR),
+    ]
+
+
+# what nk_ew_f32 evaluates: values of these types, these operations
+_EWF_TYPES = (dt.float32, dt.float16, dt.bfloat16, dt.bool_)
+_EWF_CODES = {DT_CODE[d] for d in _EWF_TYPES}
+_EWF_OPS = {OP_LOAD, OP_CONST, OP_SELECT} | set(COMPARE_CODES.values()) | {
+    UNARY_CODES[n] for n in ("negate", "abs", "exponential", "log", "sqrt", "rsqrt", "tanh", "ceil", "floor",
+                             "round_nearest_even", "trunc", "sign", "is_finite", "is_nan", "logistic", "copy")} | {
+    BINARY_CODES[n] for n in ("add", "subtract", "multiply", "divide", "maximum", "minimum")}
+_EWF_NOT = UNARY_CODES["not"]
+
+
+def collapse_dims(shape, strides):
+    """(shape, strides) with size-1 dimensions dropped and neighbours merged
+    where every operand's strides (a list per operand) allow."""
+    dims = [(int(n), [int(st[d]) for st in strides]) for d, n in enumerate(shape) if n != 1]
+    out = []
+    for n, st in dims:
+        if out and all(a == b * n for a, b in zip(out[-1][1], st)):
+            out[-1] = (out[-1][0] * n, st)
+        else:
+            out.append((n, st))
+    out = out or [(1, [0] * len(strides))]
+    return [n for n, _ in out], [[st[i] for _, st in out] for i in range(len(strides))]
+
+
 class ReduceArgs(ctypes.Structure):
     _fields_ = [
         ("inp", ctypes.c_void_p), ("out", ctypes.c_void_p),
@@ -355,8 +399,9 @@ class ProgramBuilder:
 
 
 class ProgramStep(Step):
-    """One ``nk_ew_program`` launch writing ``shape`` elements of ``out``
-    (a plain copy of a contiguous value takes the streaming copy kernel)."""
+    """One launch writing ``shape`` elements of ``out``: a plain copy of a
+    contiguous value takes the streaming copy kernel, a program over float
+    types ``nk_ew_f32`` (the same bits as) the general ``nk_ew_program``."""
 
     kind = "elementwise"
 
@@ -404,8 +449,54 @@ class ProgramStep(Step):
             nbytes = total * self.out_dtype.itemsize
             if nbytes % 16 == 0 and src % 16 == 0 and a.out % 16 == 0:
                 return [copy16(src, a.out, nbytes)]
+        fast = self._float_form(addr, total)
+        if fast is not None:
+            return [fast]
         return [Launch("generic", "nk_ew_program", (grid, 1, 1), (256, 1, 1), a,
                        bytes=total * self.out_dtype.itemsize)]
+
+
+    def _float_form(self, addr, total: int) -> Optional[Launch]:
+        """The ``nk_ew_f32`` launch, or None where a type, an operation or
+        an offset past 2^31 needs the general kernel."""
+        p = self.prog
+        if total >= 2**31 - 4096 or self.out_dtype not in _EWF_TYPES or any(
+                v.dtype not in _EWF_TYPES for v, _, _ in p.inputs):
+            return None
+        for op, _, _, _, _, dtc, flags, _ in p.instrs:
+            if dtc not in _EWF_CODES or flags or not (op in _EWF_OPS or (op == _EWF_NOT and dtc == DT_CODE[dt.bool_])):
+                return None
+        shape, strides = collapse_dims(p.shape, [self.out_strides] + [s for _, s, _ in p.inputs])
+        span = max(sum(abs(st) * (n - 1) for n, st in zip(shape, ss)) for ss in strides)
+        if span >= 2**31:
+            return None
+
+        def mode(ptr, st, isz):
+            if st[-1] == 0:
+                return 0
+            whole = st[-1] == 1 and all(x % 4 == 0 for x in st[:-1]) and ptr % (4 * isz) == 0
+            return 1 if whole else 2
+
+        a = EwfArgs()
+        a.out = addr(self.out) + self.out_offset * self.out_dtype.itemsize
+        a.total, a.rank, a.n_instr = total, len(shape), len(p.instrs)
+        a.out_dtype, a.result_reg = dtype_code(self.out_dtype), p.result
+        a.rows4 = 1 if shape[-1] % 4 == 0 else 0
+        a.out_mode = mode(a.out, strides[0], self.out_dtype.itemsize)
+        for d, n in enumerate(shape):
+            a.shape[d], a.out_strides[d] = n, strides[0][d]
+        for i, (v, _, off) in enumerate(p.inputs):
+            st = strides[1 + i]
+            a.inp[i].ptr = addr(v) + off * v.dtype.itemsize
+            for d in range(len(shape)):
+                a.inp[i].strides[d] = st[d]
+            a.inp[i].dtype, a.inp[i].mode = dtype_code(v.dtype), mode(a.inp[i].ptr, st, v.dtype.itemsize)
+        for k, (op, dst, x, y, z, dtc, _, imm) in enumerate(p.instrs):
+            I = a.prog[k]
+            I.op, I.dst, I.a, I.b, I.c, I.dtype, I.imm = op, dst, x, y, z, dtc, float(np.float32(imm))
+        grid = max(1, min(-(-total // 1024), 65536))
+        a.step = grid * 1024
+        return Launch("generic", "nk_ew_f32", (grid, 1, 1), (256, 1, 1), a, bytes=total * self.out_dtype.itemsize)
 
 
 def strided_access(v: Value, materialized) -> Tuple[Value, np.ndarray, int]:
