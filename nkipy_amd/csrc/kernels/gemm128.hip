@@ -33,28 +33,38 @@
 // x 4096 43.0 -> 36.9 us, K 14336, 128 x 4096 126 -> 102.  With two workgroups
 // per CU the four-wave form is the faster one (2000 x 4096 65 against 73).
 //
+// Few rows (_kh64, _kh32: at most 64 / 32 rows, one tile row): the same eight
+// waves over 64 or 32 rows (2 or 1 MFMA row tiles per wave).  24 rows padded to
+// 128 leave the matrix pipes, not the weight stream, as the bound (0.55 us a
+// block, 15 KB/us a CU); the smaller tile and the deeper ring its A stage
+// leaves room for (nine 64-k blocks fp8, six bf16) put the stream back.
+//
 // K ranges (grid y, *_splitk): fp32 partial planes for the reduction of
 // gemv.hip.
 #include "gemm_common.h"
 
 typedef __attribute__((address_space(3))) uint8_t lds_b;
 
-template <bool NT, bool FP8, bool SWIGLU, typename TC, bool ROPE, bool KH>
+// MI: MFMA row tiles per wave; 4 (128 rows), with KH also 2 and 1
+template <bool NT, bool FP8, bool SWIGLU, typename TC, bool ROPE, bool KH, int MI = 4>
 __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   static_assert(NT || !FP8, "no fp8 NN form");
+  static_assert(MI == 4 || (KH && (MI == 2 || MI == 1)), "few-row tiles take the eight-wave form");
   // (RING must hold the 64 KiB the KH groups exchange)
   static_assert(!ROPE || (!SWIGLU && sizeof(TC) == 2), "the rotary epilogue writes bf16 projections");
   constexpr int NW = KH ? 8 : 4;              // waves
-  constexpr int RA = KH ? (FP8 ? 6 : 4) : 3, SA = 16384;  // A ring: blocks of 64 k
+  // A ring: blocks of 64 k (32-row tiles stage 64 rows, a move per wave)
+  constexpr int SA = MI == 4 ? 16384 : 8192;
+  constexpr int RA = KH ? (MI == 4 ? (FP8 ? 6 : 4) : (FP8 ? 9 : 6)) : 3;
   // B ring: blocks of 64 k (fp8, KH), else phases of 32 k
   constexpr int RB = KH || FP8 ? RA : 4, SB = KH && !FP8 ? 16384 : 8192;
-  constexpr int NAM = 16 / NW, NBM = SB / 1024 / NW;  // 1 KiB moves per wave: A block, B block / phase
+  constexpr int NAM = SA / 1024 / NW, NBM = SB / 1024 / NW;  // 1 KiB moves per wave: A block, B block / phase
   // KH, bf16 NT: B^T rows of 128 B, as A's
   constexpr bool BL = KH && NT && !FP8;
 
   int tm, tn;
   gemm_tile(a, tm, tn);
-  const int64_t m0 = (int64_t)tm * 128;
+  const int64_t m0 = (int64_t)tm * (32 * MI);
   const int64_t n0 = (int64_t)tn * (SWIGLU ? 64 : 128);
 
   const int lane = threadIdx.x & 63;
@@ -63,9 +73,9 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   const int wm = (wave >> 1) & 1, wn = wave & 1;
   const int l16 = lane & 15, g4 = lane >> 4;
 
-  f32x4 acc[4][4];
+  f32x4 acc[MI][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -131,12 +141,12 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
     }
   };
 
-  // Fragment offsets within a stage.  A tile i: rows 64 wm + 16 i + l16; B
+  // Fragment offsets within a stage.  A tile i: rows 16 MI wm + 16 i + l16; B
   // tile j: tile columns 32 wn + brel[j] + l16 (half j / 2).  The row swizzles
   // only see l16.  A block's second 32 k: A chunk 4 + g (offset bit 6), fp8 B
   // chunk 2 + g / 2 (offset bit 5).
   constexpr int brel[4] = {0, 16, 64, 80};
-  const uint32_t aoff = ((64 * wm + l16) * 128 + ((g4 ^ swz_a64(l16)) << 4)) ^ (kg ? 64u : 0u);
+  const uint32_t aoff = ((16 * MI * wm + l16) * 128 + ((g4 ^ swz_a64(l16)) << 4)) ^ (kg ? 64u : 0u);
   uint32_t boff;  // tile 0
   if constexpr (FP8) {
     boff = ((32 * wn + l16) * 64 + (((g4 >> 1) ^ swz_b64(l16)) << 4) + 8 * (g4 & 1)) ^ (kg ? 32u : 0u);
@@ -157,12 +167,12 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   typedef __attribute__((address_space(3))) const unsigned long long lds_u64;
   // fragments of the 32 k of half h of an A block and its B (fp8: the same
   // half of the B block)
-  auto load = [&](lds_u8 *sta, lds_u8 *stb, int h, bf16x8_t (&af)[4], bf16x8_t (&bf)[4])
+  auto load = [&](lds_u8 *sta, lds_u8 *stb, int h, bf16x8_t (&af)[MI], bf16x8_t (&bf)[4])
       __attribute__((always_inline)) {
     lds_u8 *pa = sta + (h ? aoff ^ 64u : aoff);
     lds_u8 *pb = stb + (FP8 && h ? boff ^ 32u : boff);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) af[i] = *reinterpret_cast<lds_bf16x8 *>(pa + i * 2048);
+    for (int i = 0; i < MI; ++i) af[i] = *reinterpret_cast<lds_bf16x8 *>(pa + i * 2048);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if constexpr (FP8) {
@@ -185,9 +195,9 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   };
   // C^T tiles (B fragment as the A operand): lane (g, i) of tile (i', j) holds
   // output row 16 i' + i and columns (tile column) + 4 g + 0..3
-  auto mma = [&](const bf16x8_t (&af)[4], const bf16x8_t (&bf)[4]) __attribute__((always_inline)) {
+  auto mma = [&](const bf16x8_t (&af)[MI], const bf16x8_t (&bf)[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
@@ -205,16 +215,22 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   // Phases of 32 k, q = 2 t + h (half h of block t).  Phase q reads the
   // fragments of phase q + 1 from LDS while its own, read a phase earlier, feed
   // the MFMAs.
-  bf16x8_t af[2][4], bf[2][4];
+  bf16x8_t af[2][MI], bf[2][4];
   int sa = 0;  // ring slot of block t (fp8: of its B block too)
   auto next = [](int s) __attribute__((always_inline)) { return s == RA - 1 ? 0 : s + 1; };
   if constexpr (KH) {
     // the two groups of four waves take alternate 32 k of every block; block
     // t + 1's fragments are read while block t's feed the MFMAs, and block t +
-    // RA moves into the slot whose fragments are in registers
+    // RA moves into the slot whose fragments are in registers.  A SwiGLU pair over NT weights: tile column tn starts at its own place
+    // in K and wraps around.  Its tiles run one K loop each in step, and rows a
+    // power of two apart at the same k sit on the same memory channels (24 rows
+    // of 2 x 14336 x 4096 fp8: 31.0 us in step, 28.4 spread; with K ranges, which
+    // spread by themselves, 3% slower).
+    const int rot = NT && SWIGLU ? (int)((int64_t)tn * nblk / a.tiles_n) : 0;
     auto issue = [&](int t, int st) __attribute__((always_inline)) {
-      issue_a(st, (int64_t)t * 64);
-      issue_b(st, (int64_t)t * 64);
+      const int u = NT && SWIGLU && t < nblk ? (t + rot < nblk ? t + rot : t + rot - nblk) : t;
+      issue_a(st, (int64_t)u * 64);
+      issue_b(st, (int64_t)u * 64);
     };
 #pragma unroll
     for (int t = 0; t < RA; ++t) issue(t, t);
@@ -292,36 +308,38 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   }
   wait_vmem();  // no LDS DMA outlives the workgroup
   // KH: the groups add their halves' sums through the (idle) ring, group g
-  // keeping A tiles 2 g and 2 g + 1
-  constexpr int NI = KH ? 2 : 4;
+  // keeping the g-th half of the A tiles (one tile: group 0 keeps it)
+  constexpr int NI = KH && MI > 1 ? MI / 2 : MI;
   f32x4 out[NI][4];
   if constexpr (KH) {
     typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
     sync(Int<0>{});
     lds_f32x4 *X = (lds_f32x4 *)RING + (threadIdx.x & 255);
+    constexpr int HI = MI > 1 ? NI : 0;  // first tile of group 1
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) X[((kg * 2 + i) * 4 + j) * 256] = kg ? acc[i][j] : acc[2 + i][j];
+      for (int j = 0; j < 4; ++j) X[((kg * NI + i) * 4 + j) * 256] = kg ? acc[i][j] : acc[HI + i][j];
     sync(Int<0>{});
+    if (MI == 1 && kg) return;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 o = X[(((1 - kg) * 2 + i) * 4 + j) * 256];
+        const f32x4 o = X[(((1 - kg) * NI + i) * 4 + j) * 256];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) out[i][j][e] = (kg ? acc[2 + i][j][e] : acc[i][j][e]) + o[e];
+        for (int e = 0; e < 4; ++e) out[i][j][e] = (kg ? acc[HI + i][j][e] : acc[i][j][e]) + o[e];
       }
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) out[i][j] = acc[i][j];
   }
 
-  // ---- epilogue: rows 64 wm + 16 i + l16, columns 32 wn + brel[j] + 4 g ..
+  // ---- epilogue: rows 16 MI wm + 16 i + l16, columns 32 wn + brel[j] + 4 g ..
   const bool vec = (a.flags & GEMM_VEC) != 0;
-  const int64_t rbase = m0 + 64 * wm + 32 * kg + l16;
+  const int64_t rbase = m0 + 16 * MI * wm + (MI > 1 ? 8 * MI * kg : 0) + l16;
   auto put4 = [&](int64_t row, int64_t col, const float (&v)[4]) __attribute__((always_inline)) {
     if (vec && col + 3 < a.N) {
       OutT<TC>::store4(a.C, row * a.ldc + col, v);
@@ -442,13 +460,20 @@ __device__ __forceinline__ void gemm128_body(const GemmArgs &a) {
   }
 }
 
-// each with four waves (two workgroups per CU) and with eight (_kh)
+// each with four waves (two workgroups per CU) and with eight (_kh; _kh64 and
+// _kh32 for at most 64 and 32 rows)
 #define NK_GEMM128(NT, FP8, SW, TC, ROPE, name)                                    \
   extern "C" __global__ __launch_bounds__(256, 2) void name(GemmArgs a) {          \
     gemm128_body<NT, FP8, SW, TC, ROPE, false>(a);                                 \
   }                                                                                \
   extern "C" __global__ __launch_bounds__(512, 1) void name##_kh(GemmArgs a) {   \
     gemm128_body<NT, FP8, SW, TC, ROPE, true>(a);                                  \
+  }                                                                                \
+  extern "C" __global__ __launch_bounds__(512, 1) void name##_kh64(GemmArgs a) {   \
+    gemm128_body<NT, FP8, SW, TC, ROPE, true, 2>(a);                               \
+  }                                                                                \
+  extern "C" __global__ __launch_bounds__(512, 1) void name##_kh32(GemmArgs a) {   \
+    gemm128_body<NT, FP8, SW, TC, ROPE, true, 1>(a);                               \
   }
 NK_GEMM128(false, false, false, bf16, false, nk_gemm128_nn_bf16_bf16)
 NK_GEMM128(false, false, false, float, false, nk_gemm128_nn_bf16_f32)
@@ -482,13 +507,20 @@ __device__ __forceinline__ GemmArgs splitk_args(const GemmArgs &a) {
   return s;
 }
 
-// (the eight-wave form under the 8-wave kernels' names)
-#define NK_GEMM128_SPLITK(NT, FP8, tag)                                                          \
-  extern "C" __global__ __launch_bounds__(256, 2) void nk_gemm128_##tag##_f32_splitk(GemmArgs a) { \
-    gemm128_body<NT, FP8, false, float, false, false>(splitk_args<NT, FP8 ? 1 : 2>(a));          \
-  }                                                                                              \
-  extern "C" __global__ __launch_bounds__(512, 1) void nk_gemm8k_##tag##_f32_splitk(GemmArgs a) {  \
-    gemm128_body<NT, FP8, false, float, false, true>(splitk_args<NT, FP8 ? 1 : 2>(a));           \
+// (the eight-wave forms under the 8-wave kernels' names: for at most 64 rows
+// without a suffix)
+#define NK_GEMM128_SPLITK(NT, FP8, tag)                                                              \
+  extern "C" __global__ __launch_bounds__(256, 2) void nk_gemm128_##tag##_f32_splitk(GemmArgs a) {   \
+    gemm128_body<NT, FP8, false, float, false, false>(splitk_args<NT, FP8 ? 1 : 2>(a));              \
+  }                                                                                                  \
+  extern "C" __global__ __launch_bounds__(512, 1) void nk_gemm8k_##tag##_f32_splitk128(GemmArgs a) {  \
+    gemm128_body<NT, FP8, false, float, false, true>(splitk_args<NT, FP8 ? 1 : 2>(a));               \
+  }                                                                                                 \
+  extern "C" __global__ __launch_bounds__(512, 1) void nk_gemm8k_##tag##_f32_splitk(GemmArgs a) {     \
+    gemm128_body<NT, FP8, false, float, false, true, 2>(splitk_args<NT, FP8 ? 1 : 2>(a));            \
+  }                                                                                                 \
+  extern "C" __global__ __launch_bounds__(512, 1) void nk_gemm8k_##tag##_f32_splitk32(GemmArgs a) {   \
+    gemm128_body<NT, FP8, false, float, false, true, 1>(splitk_args<NT, FP8 ? 1 : 2>(a));            \
   }
 NK_GEMM128_SPLITK(false, false, nn_bf16)
 NK_GEMM128_SPLITK(true, false, nt_bf16)

@@ -296,7 +296,8 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
     aligned 16-byte row chunks) writes the output tile through LDS so that
     every global store covers whole lines.  ``tile`` 128 selects the kernels
     of 128 x 128 output tiles (gemm128.hip; no fp8 NN form, none of the other
-    options), ``kh`` their eight-wave form (default: at most 256 tiles).
+    options), ``kh`` their eight-wave form (default: at most 256 tiles), 64 or
+    32 its few-row form for that many rows (default: wherever M fits).
     """
     if layout not in ("nn", "nt"):
         raise LaunchError(f"unknown GEMM layout {layout}")
@@ -386,10 +387,10 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
         args.group_m = GEMM128_GROUP_M
         symbol = (f"nk_gemm128_swiglu_{layout}_{btag}_bf16" if swiglu else
                   f"nk_gemm128_{layout}_{btag}_{ctag}" + ("_rope" if rope is not None else ""))
-        kh = kh if kh is not None else tiles_m * tiles_n <= 256
-        symbol += "_kh" if kh else ""
-        return Launch("gemm128", symbol, (tiles_m * tiles_n, 1, 1), (512 if kh else 256, 1, 1), args, bytes=nbytes,
-                      flops=2 * M * N * K * n_mm)
+        kh = _gemm128_kh(kh, M, tiles_m * tiles_n)
+        symbol += f"_kh{kh or ''}" if kh is not None else ""
+        return Launch("gemm128", symbol, (tiles_m * tiles_n, 1, 1), (256 if kh is None else 512, 1, 1), args,
+                      bytes=nbytes, flops=2 * M * N * K * n_mm)
     has_pp = not (fp8 and layout == "nn")
     if pingpong is None:
         pingpong = has_pp
@@ -419,6 +420,22 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
                   bytes=nbytes, flops=2 * M * N * K * n_mm)
 
 
+def _gemm128_kh(kh, M: int, workgroups: int):
+    """The form of the 128-tile kernels: None four waves, 0 eight waves over
+    128 rows, 64 / 32 eight waves over that many rows.  ``kh`` None picks."""
+    if kh is None:
+        if M <= 64:
+            return 32 if M <= 32 else 64
+        return 0 if workgroups <= 256 else None
+    if kh is False:
+        return None
+    if kh is True:
+        return 0
+    if kh not in (32, 64) or M > kh:
+        raise LaunchError(f"few-row GEMM tiles take up to 32 or 64 rows, got {kh} for {M}")
+    return kh
+
+
 REDUCE4_MIN = 1 << 17
 SPLITK_TARGET_WGS = 256  # one 8-wave GEMM workgroup per CU
 
@@ -445,6 +462,12 @@ def gemm_splitk_split(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = 
 # 128 tiles in the eight-wave form; 512 of them in the four-wave form, two per
 # CU, in half rounds.  By weights: fp8 NT, bf16 NT, bf16 NN.
 _GEMM_US = {("nt", True): (20.3, 6.6, 14.6), ("nt", False): (23.5, 8.4, 17.2), ("nn", False): (20.0, 9.2, 16.5)}
+# the few-row form (at most 64 rows): a round's fixed time, its us per 1000 k, the
+# rate its weights stream at (the two add as a 3-norm: 4096 x 14336 fp8 in 5 / 6 /
+# 8 ranges 21.2 / 19.7 / 18.0 us so, measured 21.9 / 20.0 / 17.8) and the
+# reduction of its ranges
+_GEMM_FEW_ROUND, _GEMM_FEW_STREAM, _GEMM_FEW_REDUCE = 5.2, 5.2e6, 4.0
+_GEMM_FEW_US = {("nt", True): 4.9, ("nt", False): 6.5, ("nn", False): 6.4}
 _GEMM_FIXED_US = 6.0      # launch, prologue, epilogue
 _GEMM_STREAM = 4.5e6      # weight bytes per us a short product streams at
 _PLANES_RATE = 5.0e6      # partial-sum bytes per us, written and read again
@@ -461,7 +484,7 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
     idle or padded (fp8, K 4096: 1000 x 6144 58 against 86 us, 1000 x 4096 37
     against 85), and those over K ranges where they still do (300 x 4096 x
     14336 fp8: 61 us in two ranges, 101 in one, 274 on the large tiles; 24
-    rows 24 us in eight ranges).  Ranges cost their fp32 planes written and
+    rows 22 us in eight ranges).  Ranges cost their fp32 planes written and
     read once, and a second launch.  ``ranges`` False: one K loop per tile."""
     if fp8 and layout == "nn":
         return GEMM_BM, 1, K
@@ -479,6 +502,15 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
             continue
         # a SwiGLU pair in ranges runs as two launches, gate and up
         wgs = -(-M // 128) * (-(-N // 64) if swiglu and ks == 1 else -(-N // 128)) * ks
+        if M <= 64:
+            rounds, few = -(-wgs // 256), n_mm if ks > 1 else 1
+            weights = n_mm / few * N * K * (1 if fp8 else 2) / _GEMM_FEW_STREAM
+            us = few * (rounds * _GEMM_FEW_ROUND + (
+                weights ** 3 + (rounds * _GEMM_FEW_US[(layout, fp8)] * kc / 1000) ** 3) ** (1 / 3))
+            if ks > 1:
+                us += _GEMM_FEW_REDUCE + 8 * ks * M * N * n_mm / _PLANES_RATE
+            best = min(best, (us, (128, ks, kc)))
+            continue
         us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
         if ks > 1:
             planes = 4 * ks * M * N * n_mm
@@ -547,8 +579,10 @@ def gemm_splitk(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, l
         args.flags &= GEMM_VEC
         args.ksplit, args.kc = ks, kc
         symbol, block = part.symbol + "_splitk", part.block
-        if kh if kh is not None else part.grid[0] * ks <= 256:
-            symbol, block = symbol.replace("gemm128", "gemm8k"), (512, 1, 1)
+        rows = _gemm128_kh(kh, M, part.grid[0] * ks)
+        if rows is not None:
+            symbol = symbol.replace("gemm128", "gemm8k") + {0: "128", 64: "", 32: "32"}[rows]
+            block = (512, 1, 1)
         launches.append(Launch(part.module, symbol, (part.grid[0], ks, 1), block, args,
                                bytes=M * K * 2 + N * K * b_dtype.itemsize + 4 * ks * plane,
                                flops=2 * M * N * K))
@@ -730,6 +764,22 @@ def gemv_mfma_preferred(M: int, N: int, K: int, swiglu: bool = False, layout: st
         return True
     tiles = -(-N // (128 if swiglu else 256))
     return M <= GEMV_MFMA_MAX_M and tiles * -(-K // 256) <= _GEMV_MFMA_TARGET_WGS
+
+
+def gemm_few_preferred(M: int, N: int, K: int, swiglu: bool = False, layout: str = "nn",
+                       fp8: bool = False) -> bool:
+    """Whether the GEMM's few-row tiles are the form for fp8 NT weights that
+    :func:`gemv_mfma_preferred` or :func:`gemv_preferred` take too (measured with
+    cold weights): a SwiGLU pair whose 64-column tiles reach 48 of the CUs in one
+    K loop without planes (12 rows of 2 x 14336 x 4096 27.5 against 39.3 us, 2 x
+    3072 x 1024 10.0 against 11.4; but 2 x 1536 x 2048, 24 tiles, 14.8 against
+    10.7); plain, 17 rows and more (24 of 6144 x 4096 15.4 against 20.2, of 2048
+    x 1536 10.5 against 12.2), fewer from 2^25 weights on (12 of 4096 x 14336
+    21.3 against 23.4; of 4096 x 4096 13.1 against 11.9).  One row streams
+    faster on the VALU form."""
+    if M <= 1 or layout != "nt" or not fp8:
+        return False
+    return -(-N // 64) >= 48 if swiglu else M > 16 or N * K >= 1 << 25
 
 
 def gemv_mfma_workspace_bytes(M: int, N: int, K: int, swiglu: bool = False) -> int:

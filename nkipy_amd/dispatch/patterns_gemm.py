@@ -177,15 +177,19 @@ class GemmMatch(Match):
         fp8 = w.value.dtype == dt.float8_e4m3fn
         # a projection of up to 16-32 rows: the MFMA form of the few-row
         # kernels (16-row tiles, weights streamed once)
-        mfma = (self.split_k
+        # (a short projection whose planes the next launch adds keeps that form)
+        few = (self.split_k and LA.gemm_few_preferred(M, N, K, up is not None, w.layout, fp8)
+               and (M > 16 or self.planes_consumer is None)
+               and (up is None or (up.layout == w.layout and up.value.dtype == w.value.dtype)))
+        mfma = (self.split_k and not few
                 and (up is None or (up.layout == w.layout and up.value.dtype == w.value.dtype))
                 and LA.gemv_mfma_preferred(M, N, K, up is not None, w.layout, fp8))
-        small = not mfma and LA.gemv_preferred(M, w.layout, fp8)
+        small = not mfma and not few and LA.gemv_preferred(M, w.layout, fp8)
         # any more rows: output tiles of 256 or 128, over K ranges where the
         # tiles leave CUs idle
         tile, ks_g, kc_g = LA.gemm_form(M, N, K, w.layout, fp8, up is not None, self.split_k)
         splitk = not mfma and not small and ks_g > 1
-        small = small or (not mfma and M <= LA.GEMV_MAX_M and not splitk)
+        small = small or (not mfma and not few and M <= LA.GEMV_MAX_M and not splitk)
         ws = None
         fold = False
         if mfma:

@@ -1,0 +1,30 @@
+"""Routes of fp8 projections of few rows: the GEMM's few-row tiles, the MFMA
+few-row kernels, the VALU form."""
+
+import pytest
+
+from nkipy_amd.core import dtypes as dt
+from nkipy_amd.dispatch import launchers as LA
+
+A = 1 << 20
+
+
+@pytest.mark.parametrize("M,N,K,swiglu,want", [
+    (1, 14336, 4096, True, False), (2, 14336, 4096, True, True), (64, 3072, 1024, True, True),
+    (16, 1536, 2048, True, False), (16, 4096, 4096, False, False), (2, 4096, 14336, False, True),
+    (17, 64, 64, False, True)])
+def test_few_row_tiles_preferred(M, N, K, swiglu, want):
+    assert LA.gemm_few_preferred(M, N, K, swiglu, "nt", True) is want
+    assert not LA.gemm_few_preferred(M, N, K, swiglu, "nt", False)
+    assert not LA.gemm_few_preferred(M, N, K, swiglu, "nn", True)
+
+
+@pytest.mark.parametrize("M,suffix", [(1, "_kh32"), (32, "_kh32"), (33, "_kh64"), (64, "_kh64"), (65, "_kh"),
+                                      (32768, "")])
+def test_row_tiles_follow_the_rows(M, suffix):
+    l = LA.gemm(A, A, A, M, 256, 256, layout="nt", b_dtype=dt.float8_e4m3fn, c_dtype=dt.bfloat16, scale_ptr=A,
+                tile=128)
+    assert l.symbol == "nk_gemm128_nt_e4m3_bf16" + suffix
+    with pytest.raises(LA.LaunchError):
+        LA.gemm(A, A, A, 65, 256, 256, layout="nt", b_dtype=dt.float8_e4m3fn, c_dtype=dt.bfloat16, scale_ptr=A,
+                tile=128, kh=64)

@@ -153,3 +153,35 @@ def test_reduction_forms_agree(gpu, ks, c_dtype):
             gpu.sync()
             got.append(out.numpy().tobytes())
         assert got[0] == got[1]
+
+
+@pytest.mark.parametrize("layout,bd", FORMS)
+@pytest.mark.parametrize("M,Nn,K", [(1, 8, 16), (17, 136, 80), (32, 264, 1056), (33, 128, 592), (49, 200, 640),
+                                    (64, 520, 1200)])
+def test_few_row_tiles(gpu, M, Nn, K, layout, bd):
+    """The 64- and 32-row forms: edges of the MFMA row tiles, rings shorter and
+    longer than K, plain, over ranges and as a SwiGLU pair."""
+    print(f"gemm128 few rows {layout} {dt.name(bd)} {M}x{Nn}x{K}", flush=True)
+    rng = np.random.default_rng(M + Nn + K)
+    x, w, wd, scale = _operands(rng, M, Nn, K, layout, bd)
+    _, u, ud, uscale = _operands(rng, M, Nn, K, layout, bd)
+    tx, tw, ts, tu, tus = (_dev(a) for a in (dt.to_bf16(x), wd, scale, ud, uscale))
+    g, v = (x.astype(np.float64) @ (m if layout == "nn" else m.T).astype(np.float64) for m in (w, u))
+    terms = np.abs(x).astype(np.float64) @ np.abs(w if layout == "nn" else w.T).astype(np.float64)
+    out = DeviceTensor.empty((M, Nn), dt.bfloat16)
+    kc = max(64, -(-(-(-K // 3)) // 64) * 64)
+    ks = -(-K // kc)
+    ws = DeviceTensor.empty((2, ks, M, Nn), np.float32)
+    for kh in (64, 32) if M <= 32 else (64,):
+        kw = dict(layout=layout, b_dtype=bd, c_dtype=dt.bfloat16, scale_ptr=ts.ptr if ts else 0, kh=kh)
+        pair = dict(up_ptr=tu.ptr, up_scale_ptr=tus.ptr if tus else 0, **kw)
+        for opt, ref, size in ((kw, g, terms), (pair, g / (1 + np.exp(-g)) * v, 8 * (1 + np.abs(g)) * (1 + np.abs(v)))):
+            l = LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, tile=128, **opt)
+            assert l.symbol.endswith(f"_kh{kh}")
+            l.run(gpu)
+            gpu.sync()
+            _check(dt.to_float32(out.numpy()), ref, size)
+            for l in LA.gemm_splitk(tx.ptr, tw.ptr, out.ptr, M, Nn, K, split=(ks, kc), ws_ptr=ws.ptr, **opt):
+                l.run(gpu)
+            gpu.sync()
+            _check(dt.to_float32(out.numpy()), ref, size)
