@@ -38,7 +38,10 @@ struct Runtime {
   std::set<hipModule_t> modules;
   std::set<hipEvent_t> events;
   std::set<hipGraphExec_t> graphs;
+  void *bounce = nullptr;  // pinned, kBounceBytes: small reads
 };
+
+constexpr size_t kBounceBytes = 4096;
 
 Runtime g_rt;
 std::mutex g_mu;
@@ -186,6 +189,8 @@ int nkh_shutdown(void) {
   g_rt.events.clear();
   for (auto g : g_rt.graphs) hipGraphExecDestroy(g);
   g_rt.graphs.clear();
+  if (g_rt.bounce) hipHostFree(g_rt.bounce);
+  g_rt.bounce = nullptr;
   hipStreamDestroy(g_rt.stream);
   g_rt.stream = nullptr;
   g_rt.device = -1;
@@ -296,6 +301,17 @@ int nkh_memcpy_d2h(void *dst, const void *src, size_t bytes) {
   if (rc) return rc;
   rc = check_range(src, bytes, "device-to-host read");
   if (rc) return rc;
+  // A few words (a plan's checks, a scalar) go through a pinned page: the copy
+  // then queues behind the launches instead of being staged by the driver once
+  // they are done.
+  if (bytes <= kBounceBytes) {
+    if (!g_rt.bounce) NKH_HIP(hipHostMalloc(&g_rt.bounce, kBounceBytes, hipHostMallocDefault), "hipHostMalloc");
+    NKH_HIP(hipMemcpyAsync(g_rt.bounce, src, bytes, hipMemcpyDeviceToHost, g_rt.stream),
+            "hipMemcpyAsync(D2H)");
+    NKH_HIP(hipStreamSynchronize(g_rt.stream), "hipStreamSynchronize(D2H)");
+    std::memcpy(dst, g_rt.bounce, bytes);
+    return NKH_OK;
+  }
   NKH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_rt.stream),
           "hipMemcpyAsync(D2H)");
   NKH_HIP(hipStreamSynchronize(g_rt.stream), "hipStreamSynchronize(D2H)");

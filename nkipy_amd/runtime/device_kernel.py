@@ -329,10 +329,10 @@ class DeviceKernel:
         else:
             self._execute(io, save_trace, ntff_name, graph)
         if sync:
-            get_runtime().sync()
             # words the kernels left for the host (e.g. the linear-attention
-            # operand range), checked once the execution is complete
-            self.executor.run_checks()
+            # operand range): reading them waits for the execution
+            if not self.executor.run_checks():
+                get_runtime().sync()
         if auto:
             return outputs
         return None
