@@ -14,6 +14,7 @@
 
 #include "kernels/linattn.hip"
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -28,7 +29,8 @@ struct LinAttnSplit {
   int64_t nseg, rchunks, nranges;
 };
 
-LinAttnSplit linattn_split(int64_t BH, int64_t T) {
+// Segments of at least 8 chunks, halved while workgroups are missing.
+LinAttnSplit linattn_long_split(int64_t BH, int64_t T) {
   const int64_t nchunks = T / LC;
   int64_t nseg = 1;
   while (BH * nseg < kTargetWorkgroups && nchunks % (2 * nseg) == 0 && nchunks / (2 * nseg) >= 8) nseg *= 2;
@@ -47,19 +49,58 @@ LinAttnSplit linattn_split(int64_t BH, int64_t T) {
   return {nseg, rchunks, (nseg - 1) * (cs / rchunks)};
 }
 
+// Time of a split in units of 0.05 us: the scan's 4 us and 3 us per chunk of a
+// segment, 0.8 us per partial state that the last segment adds to its start;
+// the partial-sum launch's 10.5 us and 0.75 us per chunk of a range.
+int64_t linattn_cost(int64_t BH, int64_t nchunks, const LinAttnSplit &s) {
+  auto rounds = [](int64_t wgs) { return (wgs + kTargetWorkgroups - 1) / kTargetWorkgroups; };
+  int64_t cost = rounds(BH * s.nseg) * (80 + 60 * (nchunks / s.nseg)) + 16 * s.nranges;
+  if (s.nranges) cost += 30 + rounds(BH * s.nranges) * (180 + 15 * s.rchunks);
+  return cost;
+}
+
+// The cheapest split that keeps to one workgroup per CU, where it saves a tenth
+// against the long segments (the rule of the Python launcher).
+LinAttnSplit linattn_split(int64_t BH, int64_t T) {
+  const int64_t nchunks = T / LC;
+  LinAttnSplit best = linattn_long_split(BH, T);
+  int64_t least = linattn_cost(BH, nchunks, best) * 9 / 10;
+  for (int64_t n = 2; n <= nchunks && n * BH <= kTargetWorkgroups; ++n) {
+    if (nchunks % n) continue;
+    const LinAttnSplit s{n, nchunks / n, n - 1};
+    const int64_t c = linattn_cost(BH, nchunks, s);
+    if (c < least) {
+      least = c;
+      best = s;
+    }
+  }
+  return best;
+}
+
 int64_t workspace_bytes(int64_t BH, const LinAttnSplit &s) {
   return BH * s.nranges * (int64_t)(LD + 1) * LDV * (int64_t)sizeof(float);
+}
+
+// What a call needs at least (the long segments), what it takes at most, and the
+// split that `bytes` of workspace hold.
+int64_t least_workspace(int64_t BH, int64_t T) { return workspace_bytes(BH, linattn_long_split(BH, T)); }
+int64_t full_workspace(int64_t BH, int64_t T) {
+  return std::max(least_workspace(BH, T), workspace_bytes(BH, linattn_split(BH, T)));
+}
+LinAttnSplit linattn_split_within(int64_t BH, int64_t T, size_t bytes) {
+  const LinAttnSplit s = linattn_split(BH, T);
+  return (size_t)workspace_bytes(BH, s) <= bytes ? s : linattn_long_split(BH, T);
 }
 
 int check_shape(int64_t BH, int64_t T) {
   if (BH <= 0 || T <= 0 || T % LC)
     return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention needs BH > 0 and T a positive multiple of 64, got BH=" +
                                                         std::to_string(BH) + " T=" + std::to_string(T));
-  const LinAttnSplit s = linattn_split(BH, T);
   // grid sizes, and the kernels' 32-bit byte offsets within a segment / range
-  if (BH * s.nseg >= (int64_t(1) << 31) || BH * (s.nranges > 0 ? s.nranges : 1) >= (int64_t(1) << 31) ||
-      (T / s.nseg) * LD * 2 >= (int64_t(1) << 31))
-    return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention problem too large for one launch");
+  for (const LinAttnSplit &x : {linattn_long_split(BH, T), linattn_split(BH, T)})
+    if (BH * x.nseg >= (int64_t(1) << 31) || BH * (x.nranges > 0 ? x.nranges : 1) >= (int64_t(1) << 31) ||
+        (T / x.nseg) * LD * 2 >= (int64_t(1) << 31))
+      return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention problem too large for one launch");
   return NKH_OK;
 }
 
@@ -74,9 +115,8 @@ int check_ptrs(const void *q, const void *k, const void *v, const void *o) {
 
 // Both launches on `stream`; `part` holds the partial states when the
 // sequences are segmented.
-int launch_linattn(const void *q, const void *k, const void *v, void *o, int64_t BH, int64_t T, float *part,
-                   hipStream_t stream) {
-  const LinAttnSplit s = linattn_split(BH, T);
+int launch_linattn(const void *q, const void *k, const void *v, void *o, int64_t BH, int64_t T,
+                   const LinAttnSplit &s, float *part, hipStream_t stream) {
   if (s.nranges) {
     LinAttnStateArgs sa{static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v), part, BH, T,
                         (int32_t)s.nranges, (int32_t)s.rchunks, nullptr};
@@ -136,7 +176,7 @@ int nkh_linear_attention_workspace_size(int64_t bh, int64_t t, size_t *bytes) {
   if (!bytes) return nkh_internal::set_error(NKH_ERR_INVALID, "bytes is null");
   int rc = check_shape(bh, t);
   if (rc) return rc;
-  *bytes = (size_t)workspace_bytes(bh, linattn_split(bh, t));
+  *bytes = (size_t)full_workspace(bh, t);
   return NKH_OK;
 }
 
@@ -146,16 +186,17 @@ int nkh_linear_attention(const void *q, const void *k, const void *v, void *o, i
   if (rc) return rc;
   rc = check_ptrs(q, k, v, o);
   if (rc) return rc;
-  const size_t need = (size_t)workspace_bytes(bh, linattn_split(bh, t));
+  const size_t need = (size_t)least_workspace(bh, t);
+  const LinAttnSplit split = linattn_split_within(bh, t, workspace ? workspace_size : 0);
   if (need && (!workspace || workspace_size < need))
     return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention of BH=" + std::to_string(bh) + " T=" +
                                                         std::to_string(t) + " needs a workspace of " +
                                                         std::to_string(need) + " bytes, got " +
                                                         std::to_string(workspace_size));
-  if (need && reinterpret_cast<uintptr_t>(workspace) % 16)
+  if (split.nranges && reinterpret_cast<uintptr_t>(workspace) % 16)
     return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention workspace must be 16-byte aligned");
   return nkh_internal::with_stream([&](hipStream_t stream, int) {
-    return launch_linattn(q, k, v, o, bh, t, static_cast<float *>(workspace), stream);
+    return launch_linattn(q, k, v, o, bh, t, split, static_cast<float *>(workspace), stream);
   });
 }
 
@@ -164,7 +205,8 @@ int nkh_linear_attention_noalloc(const void *q, const void *k, const void *v, vo
   if (rc) return rc;
   rc = check_ptrs(q, k, v, o);
   if (rc) return rc;
-  const size_t need = (size_t)workspace_bytes(bh, linattn_split(bh, t));
+  const size_t need = (size_t)least_workspace(bh, t);
+  const LinAttnSplit split = linattn_split_within(bh, t, NKH_NOALLOC_SCRATCH_BYTES);
   if (need > NKH_NOALLOC_SCRATCH_BYTES)
     return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention of BH=" + std::to_string(bh) + " T=" +
                                                         std::to_string(t) + " needs " + std::to_string(need) +
@@ -179,7 +221,7 @@ int nkh_linear_attention_noalloc(const void *q, const void *k, const void *v, vo
       ptr = (device >= 0 && device < kMaxDevices) ? g_scratch[device] : nullptr;
     }
     if (!ptr) return nkh_internal::set_error(NKH_ERR_NOT_INIT, "scratch of this device is not set up");
-    return launch_linattn(q, k, v, o, bh, t, static_cast<float *>(ptr), stream);
+    return launch_linattn(q, k, v, o, bh, t, split, static_cast<float *>(ptr), stream);
   });
 }
 

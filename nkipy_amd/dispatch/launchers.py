@@ -989,10 +989,9 @@ LINATTN_D = 128
 LINATTN_TARGET_WGS = 256
 
 
-def linear_attention_split(BH: int, T: int, ranges_per_segment: int = None):
-    """(segments per sequence, chunks per partial-sum range, ranges) for the
-    linear-attention scan of BH sequences of length T; ``ranges_per_segment``
-    (1, 2 or 4) overrides the partial-sum range policy."""
+def _linattn_long_split(BH: int, T: int, ranges_per_segment: int = None):
+    """The split into segments of at least 8 chunks, halved while workgroups
+    are missing."""
     nchunks = T // LINATTN_CHUNK
     nseg = 1
     while (BH * nseg < LINATTN_TARGET_WGS and nchunks % (2 * nseg) == 0
@@ -1014,14 +1013,50 @@ def linear_attention_split(BH: int, T: int, ranges_per_segment: int = None):
         rchunks = cs // 2
     else:
         rchunks = cs // 4
+    return nseg, rchunks
+
+
+def _linattn_cost(BH: int, nchunks: int, nseg: int, rchunks: int) -> int:
+    """Time of a split in units of 0.05 us: the scan's 4 us and 3 us per chunk
+    of a segment (a serial chain), 0.8 us per partial state that the last
+    segment adds to its start; the partial-sum launch's 10.5 us and 0.75 us
+    per chunk of a range (measured over 6 to 64 sequences of 256 to 8192)."""
+    cs = nchunks // nseg
     nranges = (nseg - 1) * (cs // rchunks)
-    return nseg, rchunks, nranges
+    cost = -(-BH * nseg // LINATTN_TARGET_WGS) * (80 + 60 * cs) + 16 * nranges
+    if nranges:
+        cost += 30 + -(-BH * nranges // LINATTN_TARGET_WGS) * (180 + 15 * rchunks)
+    return cost
+
+
+@functools.lru_cache(maxsize=4096)
+def linear_attention_split(BH: int, T: int, ranges_per_segment: int = None):
+    """(segments per sequence, chunks per partial-sum range, ranges) for the
+    linear-attention scan of BH sequences of length T: the cheapest split by
+    :func:`_linattn_cost` that keeps to one workgroup per CU, any divisor of
+    the chunks, where it saves a tenth against segments of at least 8 chunks;
+    ``ranges_per_segment`` (1, 2 or 4) overrides the partial-sum range policy
+    of those.  Whole calls, against those: 24 sequences of 768 in 6 segments
+    57 -> 48 us, 24 of 1536 in 8 72 -> 57, 6 of 4096 in 16 80 -> 63, 16 of 6400
+    in 10 125 -> 82, 36 of 10240 in 5 205 -> 175; 64 of 8192 keep 4."""
+    nchunks = T // LINATTN_CHUNK
+    nseg, rchunks = _linattn_long_split(BH, T, ranges_per_segment)
+    if ranges_per_segment is None:
+        best = (_linattn_cost(BH, nchunks, nseg, rchunks) * 9 // 10, nseg, rchunks)
+        for n in range(2, min(nchunks, LINATTN_TARGET_WGS // BH) + 1):
+            if nchunks % n == 0:
+                best = min(best, (_linattn_cost(BH, nchunks, n, nchunks // n), n, nchunks // n))
+        _, nseg, rchunks = best
+    return nseg, rchunks, (nseg - 1) * (nchunks // nseg // rchunks)
 
 
 def linear_attention_workspace_bytes(BH: int, T: int, ranges_per_segment: int = None) -> int:
-    """Device workspace (fp32 partial prefix states) the launch needs; 0 if
+    """Device workspace (fp32 partial prefix states) of the launch, and at
+    least that of the long segments, which the C entry point asks for; 0 if
     the sequences run unsegmented."""
     _, _, nranges = linear_attention_split(BH, T, ranges_per_segment)
+    nseg, rchunks = _linattn_long_split(BH, T, ranges_per_segment)
+    nranges = max(nranges, (nseg - 1) * (T // LINATTN_CHUNK // nseg // rchunks))
     return BH * nranges * (LINATTN_D + 1) * LINATTN_D * 4
 
 
