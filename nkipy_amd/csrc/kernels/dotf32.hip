@@ -20,6 +20,9 @@
 // a time along k (1) or along rows / columns (2) where strides, sizes and
 // alignment allow, else element by element (0); one kernel per pair of modes
 // and element widths (nk_dot_f32_<f|h><mode A>_<f|h><mode B>).
+// fp32 pairs also come over 32 x 128 tiles (the four waves side by side; 46 KiB:
+// three workgroups per CU) for up to 32 rows, which 64-row tiles pad to twice
+// the matrix work: one row of a feed-forward of 2048 / 6144 78 -> 63 us.
 // K ranges (grid z = batch x ksplit) write fp32 planes [range][batch m][n] for
 // the reduction of gemv.hip when the tiles leave CUs idle.
 #include "common.h"
@@ -42,26 +45,28 @@ struct DotF32Args {
   int32_t a_bytes, b_bytes;  // one batch's span of each operand (< 2 GiB)
 };
 
-constexpr int TS = 64, KS = 32;
-// LDS layouts: modes 0 and 1 [64 rows][32 k + 4], mode 2 as it lies in memory,
-// [32 k][64 rows + 4]: 16-byte writes, and both kinds of read (16 rows x 16
+constexpr int KS = 32;
+// LDS layouts: modes 0 and 1 [rows][32 k + 4], mode 2 as it lies in memory,
+// [32 k][rows + 4]: 16-byte writes, and both kinds of read (16 rows x 16
 // bytes, 16 rows x four k) spread over all banks
-constexpr int PITCH = KS + 4, KPITCH = TS + 4;
+constexpr int PITCH = KS + 4;
 constexpr uint32_t FAR = 0x80000000u;  // past every operand (each spans less than 2 GiB): reads zeros
 
-// One operand's stage (64 rows x 32 k): this thread's two 4-element pieces as
-// raw words.  MODE 1: row t / 8 + 32 u, k 4 (t % 8); MODE 2: k t / 16 + 16 u,
-// rows 4 (t % 16); MODE 0: as MODE 1, element by element.  HALF: 16-bit
+// One operand's stage (R rows x 32 k): this thread's R / 32 4-element pieces as
+// raw words.  MODE 1: row t / 8 + 32 u, k 4 (t % 8); MODE 2 (64 rows): k t / 16
+// + 16 u, rows 4 (t % 16); MODE 0: as MODE 1, element by element.  HALF: 16-bit
 // elements.  Loads go through a buffer resource with out-of-range pieces sent
 // past its end, so no load sits behind a branch and all stay in flight until
 // the pieces are widened on their way into LDS.
-template <int MODE, bool HALF>
+template <int MODE, bool HALF, int ROWS>
 struct Operand {
   static constexpr int ES = HALF ? 2 : 4;
+  static constexpr int U = ROWS / 32, R4 = ROWS / 4, KSTEP = 256 / R4, KPITCH = ROWS + 4;
+  static constexpr int WORDS = ROWS * PITCH > KS * KPITCH ? ROWS * PITCH : KS * KPITCH;
   __amdgpu_buffer_rsrc_t r;
-  uint32_t off[2], kstep, estep;
-  int kofs[2], dt;
-  uint32_t w[2][4];
+  uint32_t off[U], kstep, estep;
+  int kofs[U], dt;
+  uint32_t w[U][4];
 
   __device__ __forceinline__ void init(const void *p, int64_t bytes, int dtype, int64_t r0, int64_t R, int64_t sr,
                                        int64_t sk) {
@@ -71,9 +76,9 @@ struct Operand {
     kstep = (uint32_t)(sk * ES);
     estep = (uint32_t)((MODE == 2 ? sr : sk) * ES);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int64_t row = r0 + (MODE == 2 ? 4 * (t & 15) : (t >> 3) + 32 * u);
-      kofs[u] = MODE == 2 ? (t >> 4) + 16 * u : 4 * (t & 7);
+    for (int u = 0; u < U; ++u) {
+      const int64_t row = r0 + (MODE == 2 ? 4 * (t % R4) : (t >> 3) + 32 * u);
+      kofs[u] = MODE == 2 ? t / R4 + KSTEP * u : 4 * (t & 7);
       off[u] = row < R ? (uint32_t)((row * sr + kofs[u] * sk) * ES) : FAR;
     }
   }
@@ -81,7 +86,7 @@ struct Operand {
   __device__ __forceinline__ void fetch(int64_t k0, int64_t k1) {
     const uint32_t so = __builtin_amdgcn_readfirstlane((uint32_t)k0 * kstep);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       if constexpr (MODE == 0) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -106,7 +111,7 @@ struct Operand {
   __device__ __forceinline__ void put(float *S) const {
     const int t = threadIdx.x;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       f32x4_t v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -118,7 +123,7 @@ struct Operand {
         }
       }
       if constexpr (MODE == 2) {
-        *reinterpret_cast<f32x4_t *>(S + ((t >> 4) + 16 * u) * KPITCH + 4 * (t & 15)) = v;
+        *reinterpret_cast<f32x4_t *>(S + (t / R4 + KSTEP * u) * KPITCH + 4 * (t % R4)) = v;
       } else {
         *reinterpret_cast<f32x4_t *>(S + ((t >> 3) + 32 * u) * PITCH + 4 * (t & 7)) = v;
       }
@@ -137,17 +142,21 @@ struct Operand {
   }
 };
 
-template <int MA, bool HA, int MB, bool HB>
+// TM x TN: 64 x 64 (waves 2 x 2) or 32 x 128 (waves 1 x 4)
+template <int MA, bool HA, int MB, bool HB, int TM, int TN>
 __device__ __forceinline__ void dot_f32_body(const DotF32Args &a) {
-  __shared__ __attribute__((aligned(16))) float SA[2][TS * PITCH], SB[2][TS * PITCH];
+  using OpA = Operand<MA, HA, TM>;
+  using OpB = Operand<MB, HB, TN>;
+  __shared__ __attribute__((aligned(16))) float SA[2][OpA::WORDS], SB[2][OpB::WORDS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, g = lane >> 4;
+  constexpr int WN = TN / 32;
+  const int wm = wave / WN, wn = wave % WN, l16 = lane & 15, g = lane >> 4;
   const int64_t b = blockIdx.z / (uint32_t)a.ksplit;
   const int sp = blockIdx.z % (uint32_t)a.ksplit;
-  const int64_t m0 = (int64_t)blockIdx.y * TS, n0 = (int64_t)blockIdx.x * TS;
+  const int64_t m0 = (int64_t)blockIdx.y * TM, n0 = (int64_t)blockIdx.x * TN;
   const int64_t k0 = (int64_t)sp * a.kc, k1 = min(k0 + a.kc, a.K);
-  Operand<MA, HA> oa;
-  Operand<MB, HB> ob;
+  OpA oa;
+  OpB ob;
   oa.init((const uint8_t *)a.A + b * a.sab * oa.ES, a.a_bytes, a.a_dtype, m0, a.M, a.sam, a.sak);
   ob.init((const uint8_t *)a.B + b * a.sbb * ob.ES, a.b_bytes, a.b_dtype, n0, a.N, a.sbn, a.sbk);
 
@@ -215,7 +224,7 @@ __device__ __forceinline__ void dot_f32_body(const DotF32Args &a) {
 
 #define NK_DOT(MA, ta, HA, MB, tb, HB)                                                               \
   extern "C" __global__ __launch_bounds__(256, 4) void nk_dot_f32_##ta##MA##_##tb##MB(DotF32Args a) { \
-    dot_f32_body<MA, HA, MB, HB>(a);                                                                 \
+    dot_f32_body<MA, HA, MB, HB, 64, 64>(a);                                                              \
   }
 #define NK_DOT_B(MA, ta, HA)                                                           \
   NK_DOT(MA, ta, HA, 0, f, false) NK_DOT(MA, ta, HA, 1, f, false) NK_DOT(MA, ta, HA, 2, f, false) \
@@ -226,3 +235,10 @@ NK_DOT_B(2, f, false)
 NK_DOT_B(0, h, true)
 NK_DOT_B(1, h, true)
 NK_DOT_B(2, h, true)
+#define NK_DOT_WIDE(MA, MB)                                                                            \
+  extern "C" __global__ __launch_bounds__(256, 3) void nk_dot_f32_f##MA##_f##MB##_wide(DotF32Args a) { \
+    dot_f32_body<MA, false, MB, false, 32, 128>(a);                                                    \
+  }
+NK_DOT_WIDE(0, 0) NK_DOT_WIDE(0, 1) NK_DOT_WIDE(0, 2)
+NK_DOT_WIDE(1, 0) NK_DOT_WIDE(1, 1) NK_DOT_WIDE(1, 2)
+NK_DOT_WIDE(2, 0) NK_DOT_WIDE(2, 1) NK_DOT_WIDE(2, 2)

@@ -581,18 +581,26 @@ class DotF32Args(ctypes.Structure):
 
 
 _DOT_F32 = {dt.float32: 0, dt.float16: 1, dt.bfloat16: 2}
-DOT_TILE = 64
+DOT_TILE = 128  # the larger side of a tile
 DOT_TARGET_WGS = 768  # three workgroups per CU
 DOT_MIN_RANGE = 128   # k per range
 
 
-def dot_split(batch: int, M: int, N: int, K: int) -> Tuple[int, int]:
+def dot_tile(M: int, N: int, fp32: bool) -> Tuple[int, int]:
+    """Tile of :class:`DotStep`'s matrix-core form: 32 x 128 for fp32 pairs of
+    up to 32 rows (feed-forwards of 2048 / 6144, us against 64 x 64: 1 row 63 /
+    78, 9 rows 66 / 82; from 33 rows on they are no faster even where they pad
+    less: 100 rows 133 / 132, 200 rows 236 / 225, 600 rows 569 / 517)."""
+    return (32, 128) if fp32 and M <= 32 and N > 64 else (64, 64)
+
+
+def dot_split(batch: int, M: int, N: int, K: int, tile: Tuple[int, int] = (64, 64)) -> Tuple[int, int]:
     """(ranges, k per range) of :class:`DotStep`'s matrix-core form: K ranges
     when the tiles alone do not give every CU three workgroups (us, one range
     / as many as do: 200 x 1024 x 3072 101 / 24, 200 x 6144 x 1024 45 / 38, 1
     x 2048 x 8192 276 / 24; 1024 x 3072 x 1024, 768 tiles, 59 in one, 66 in
     two), of 128 k at least."""
-    tiles = batch * -(-M // DOT_TILE) * -(-N // DOT_TILE)
+    tiles = batch * -(-M // tile[0]) * -(-N // tile[1])
     ks = max(1, min(DOT_TARGET_WGS // tiles, K // DOT_MIN_RANGE, 65535 // batch))
     while ks > 1 and 4 * ks * batch * M * N > 1 << 27:
         ks -= 1
@@ -669,9 +677,10 @@ class DotStep(Step):
         self.f32 = all(v.dtype in _DOT_F32 for v in (a_v, b_v, node.out)) and span < 2**31
         self.split, self.planes = (1, self.K), None
         outputs = self.batch * self.M * self.N
+        self.tile = dot_tile(self.M, self.N, a_v.dtype == dt.float32 and b_v.dtype == dt.float32)
         if self.f32 and plan is not None and outputs > 0:
             # (the reduction writes fp32 or bf16)
-            ks, kc = dot_split(self.batch, self.M, self.N, self.K)
+            ks, kc = dot_split(self.batch, self.M, self.N, self.K, self.tile)
             if ks > 1 and node.out.dtype != dt.float16 and outputs < 2**31:
                 self.split = ks, kc
                 self.planes = Slot(plan.add_buffer(4 * ks * outputs, "temp", "dot.partials"))
@@ -697,7 +706,9 @@ class DotStep(Step):
         a.c_vec = 1 if a.c_dtype == 0 and self.N % 4 == 0 and a.C % 16 == 0 else 0
         rows = self.batch * self.M
         sym = f"nk_dot_f32_{'f' if esa == 4 else 'h'}{a.a_mode}_{'f' if esb == 4 else 'h'}{a.b_mode}"
-        ls = [Launch("dotf32", sym, (-(-self.N // DOT_TILE), -(-self.M // DOT_TILE), self.batch * ks),
+        tm, tn = self.tile
+        sym += "_wide" if tm == 32 else ""
+        ls = [Launch("dotf32", sym, (-(-self.N // tn), -(-self.M // tm), self.batch * ks),
                      (256, 1, 1), a, flops=2 * rows * self.N * self.K)]
         if ks > 1:
             red = GemvArgs(None, None, None, out, None, None, None, None, a.C, rows, self.N, self.K, self.K, self.K,

@@ -87,3 +87,21 @@ def test_ranges_and_load_modes():
     assert G._dot_mode(256, 2, 64, 2, 0, 10, 64, 1) == 0
     assert G._dot_mode(256, 4, 65, 1, 0, 1, 64, 1) == 1
     assert G._dot_span(4, 64, 1, 10, 64) == 4 * 640 and G._dot_span(4, -64, 1, 10, 64) > 2**31
+
+
+WIDE = [(1, 1, 128, 32), (2, 17, 130, 257), (1, 32, 384, 64), (3, 5, 900, 31), (1, 9, 65, 1100)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("batch,M,N,K", WIDE)
+def test_wide_tiles_match_float64(gpu, form, batch, M, N, K):
+    """Sizes the 32 x 128 tiles take (fp32 pairs): every load mode, edges of
+    both sides, ranges."""
+    test_products_match_float64(gpu, form, batch, M, N, K, ("float32", "float32"))
+
+
+def test_tile_choice():
+    assert all(G.dot_tile(M, N, True) == (32, 128) for _, M, N, _ in WIDE)
+    assert G.dot_tile(2, 1024, False) == (64, 64) and G.dot_tile(1, 64, True) == (64, 64)
+    assert G.dot_tile(33, 4096, True) == (64, 64)
