@@ -452,6 +452,69 @@ extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// SwiGLU over a fp32 product's partial planes: with P the sum of the planes in
+// the order of gemv.hip's reduction (four interleaved sums), out[m][j] = (g * (1 / (1 + exp(-g)))) * u, g = P[m][og + j], u = P[m][ou
+// + j].  The planes' reduction and the program of nk_ew_f32 in one launch, bit
+// for bit theirs (fp32 values, exp rounded from double).  Latency bounds the
+// small sizes, of which the interpreter's decode and dependent loads were most;
+// all loads of a thread's four outputs are in flight together here.  200 x 3072
+// from two planes 5.0 us, the two launches it replaces 4.9 + 9.3; 2 x 3072
+// from eight 4.0, 4.0 + 8.9.
+// ---------------------------------------------------------------------------
+struct SwigluPlanesArgs {
+  const float *P;
+  float *out;
+  int64_t plane;  // elements of a plane
+  int32_t rows, F, N, ks, og, ou;
+};
+extern "C" __global__ __launch_bounds__(64) void nk_swiglu_planes_f32(SwigluPlanesArgs a) {
+  const uint32_t i = blockIdx.x * 64 + threadIdx.x, f4 = (uint32_t)a.F / 4;
+  const uint32_t r = i / f4, j = 4 * (i % f4);
+  if (r >= (uint32_t)a.rows) return;
+  const float *p = a.P + (int64_t)r * a.N + j;
+  float g4[4][4], u4[4][4];  // (0 + x is x but for x = -0: one plane is copied)
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) g4[q][e] = u4[q][e] = 0.f;
+  for (int s0 = 0; s0 < a.ks; s0 += 4) {
+    float4 x[4], y[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t s = min(s0 + q, a.ks - 1) * a.plane;
+      x[q] = *reinterpret_cast<const float4 *>(p + s + a.og);
+      y[q] = *reinterpret_cast<const float4 *>(p + s + a.ou);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (s0 + q >= a.ks) break;
+      const float xv[4] = {x[q].x, x[q].y, x[q].z, x[q].w}, yv[4] = {y[q].x, y[q].y, y[q].z, y[q].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        g4[q][e] = a.ks == 1 ? xv[e] : g4[q][e] + xv[e];
+        u4[q][e] = a.ks == 1 ? yv[e] : u4[q][e] + yv[e];
+      }
+    }
+  }
+  float g[4], u[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    g[e] = a.ks == 1 ? g4[0][e] : (g4[0][e] + g4[1][e]) + (g4[2][e] + g4[3][e]);
+    u[e] = a.ks == 1 ? u4[0][e] : (u4[0][e] + u4[1][e]) + (u4[2][e] + u4[3][e]);
+  }
+  float o[4];
+  {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = 1.f + (float)exp((double)-g[e]);
+      o[e] = g[e] * (1.f / d) * u[e];
+    }
+  }
+  *reinterpret_cast<float4 *>(a.out + (int64_t)r * a.F + j) = make_float4(o[0], o[1], o[2], o[3]);
+}
+
+// ---------------------------------------------------------------------------
 // Reduction: one workgroup per output element.
 // ---------------------------------------------------------------------------
 #define RED_MAX_RANK 6

@@ -676,6 +676,7 @@ class DotStep(Step):
                    _dot_span(b_v.dtype.itemsize, self.sbn, self.sbk, self.N + DOT_TILE, self.K + 2 * DOT_TILE))
         self.f32 = all(v.dtype in _DOT_F32 for v in (a_v, b_v, node.out)) and span < 2**31
         self.split, self.planes = (1, self.K), None
+        self.keep_planes = False  # the consumer adds them (SwigluPlanesStep)
         outputs = self.batch * self.M * self.N
         self.tile = dot_tile(self.M, self.N, a_v.dtype == dt.float32 and b_v.dtype == dt.float32)
         if self.f32 and plan is not None and outputs > 0:
@@ -704,17 +705,20 @@ class DotStep(Step):
         a.b_bytes = _dot_span(esb, self.sbn, self.sbk, self.N, self.K)
         a.ksplit, a.kc = ks, kc if ks > 1 else -(-max(self.K, 1) // 32) * 32
         a.c_vec = 1 if a.c_dtype == 0 and self.N % 4 == 0 and a.C % 16 == 0 else 0
-        rows = self.batch * self.M
         sym = f"nk_dot_f32_{'f' if esa == 4 else 'h'}{a.a_mode}_{'f' if esb == 4 else 'h'}{a.b_mode}"
         tm, tn = self.tile
         sym += "_wide" if tm == 32 else ""
         ls = [Launch("dotf32", sym, (-(-self.N // tn), -(-self.M // tm), self.batch * ks),
-                     (256, 1, 1), a, flops=2 * rows * self.N * self.K)]
-        if ks > 1:
-            red = GemvArgs(None, None, None, out, None, None, None, None, a.C, rows, self.N, self.K, self.K, self.K,
-                           self.N, ks, kc, 0, 0)
-            ls.append(_reduce_planes(red, ctype, False))
-        return ls
+                     (256, 1, 1), a, flops=2 * self.batch * self.M * self.N * self.K)]
+        return ls + ([] if self.keep_planes else self.reduction(addr))
+
+    def reduction(self, addr):
+        ks, kc = self.split
+        if ks == 1:
+            return []
+        red = GemvArgs(None, None, None, addr(self.node.out), None, None, None, None, addr(self.planes),
+                       self.batch * self.M, self.N, self.K, self.K, self.K, self.N, ks, kc, 0, 0)
+        return [_reduce_planes(red, self.node.out.dtype, False)]
 
     def launches(self, addr):
         if self.M * self.N * self.batch == 0:
@@ -736,6 +740,100 @@ class DotStep(Step):
         a.c_dtype = dtype_code(self.node.out.dtype)
         return [Launch("generic", "nk_dot", (gx, gy, self.batch), (256, 1, 1), a,
                        flops=2 * self.batch * self.M * self.N * self.K)]
+
+
+class SwigluPlanesArgs(ctypes.Structure):
+    _fields_ = [("P", ctypes.c_void_p), ("out", ctypes.c_void_p), ("plane", ctypes.c_int64)] + \
+        [(n, ctypes.c_int32) for n in ("rows", "F", "N", "ks", "og", "ou")]
+
+
+class SwigluPlanesStep(Step):
+    """``(g * (1 / (1 + exp(-g)))) * u`` over two column blocks of a fp32
+    product that nothing else reads, from the product's partial planes
+    (nk_swiglu_planes_f32): one launch for the planes' reduction and the
+    program, the same bits."""
+
+    kind = "swiglu"
+
+    def __init__(self, dot: DotStep, prog: ProgramStep, cols: Tuple[int, int]):
+        super().__init__("SwiGLU of a product's planes", prog.inputs, prog.outputs)
+        self.dot, self.prog, self.cols = dot, prog, cols
+
+    def launches(self, addr):
+        d = self.dot
+        out, ks = addr(self.prog.out), d.split[0]
+        part = addr(d.planes) if ks > 1 else addr(d.node.out)
+        if out % 16 or part % 16:
+            return d.reduction(addr) + self.prog.launches(addr)
+        rows, F = d.batch * d.M, self.prog.prog.shape[-1]
+        if rows * F == 0:
+            return []
+        a = SwigluPlanesArgs(part, out, rows * d.N, rows, F, d.N, ks, *self.cols)
+        return [Launch("generic", "nk_swiglu_planes_f32", (-(-rows * F // 256), 1, 1), (64, 1, 1), a,
+                       bytes=4 * rows * F * (2 * ks + 1))]
+
+
+def _swiglu_columns(prog: Program, v: Value) -> Optional[Tuple[int, int]]:
+    """(first gate column, first up column) when the program is the SwiGLU of
+    two column blocks of ``v``, else None."""
+    code = dtype_code(dt.float32)
+    regs: Dict[int, tuple] = {}
+    exp, neg = UNARY_CODES["exponential"], UNARY_CODES["negate"]
+    add, mul, div = (BINARY_CODES[n] for n in ("add", "multiply", "divide"))
+    for op, dst, x, y, _, dtc, flags, imm in prog.instrs:
+        if dtc != code or flags:
+            return None
+        if op == OP_LOAD:
+            regs[dst] = ("load", int(imm))
+        elif op == OP_CONST:
+            regs[dst] = ("const", imm)
+        elif op in (exp, neg):
+            regs[dst] = (op, regs[x])
+        elif op in (add, mul, div):
+            ab = (regs[x], regs[y])
+            regs[dst] = (op,) + (ab if op == div else tuple(sorted(ab, key=repr)))
+        else:
+            return None
+    pair = lambda op, *ab: (op,) + tuple(sorted(ab, key=repr))
+    one = ("const", 1.0)
+    silu = lambda g: pair(mul, g, (div, one, pair(add, one, (exp, (neg, g)))))
+    if len(prog.inputs) != 2:
+        return None
+    lead = tuple(int(s) for s in contiguous_strides(v.shape))
+    offs = []
+    for w, strides, off in prog.inputs:
+        if w.id != v.id or tuple(strides) != lead or off % 4 or off < 0 or off + prog.shape[-1] > v.shape[-1]:
+            return None
+        offs.append(off)
+    for g, u in ((0, 1), (1, 0)):
+        if regs[prog.result] == pair(mul, silu(("load", g)), ("load", u)):
+            return offs[g], offs[u]
+    return None
+
+
+def fuse_swiglu_planes(plan):
+    """Replace the programs that are a SwiGLU over a fp32 product's planes."""
+    buffer = lambda v: plan.slots[v.id].buffer if v.id in plan.slots else None
+    for i, st in enumerate(plan.steps):
+        if not isinstance(st, ProgramStep) or not st.prog.inputs or st.out.dtype != dt.float32:
+            continue
+        v = st.prog.inputs[0][0]
+        dots = [d for d in plan.steps[:i] if isinstance(d, DotStep) and d.node.out.id == v.id]
+        if len(dots) != 1 or not dots[0].f32 or v.dtype != dt.float32 or buffer(v) is None:
+            continue
+        d, p = dots[0], st.prog
+        if (plan.buffers[buffer(v)].kind != "temp" or d.N != v.shape[-1] or d.N % 4 or len(p.shape) != v.ndim
+                or p.shape[:-1] != tuple(v.shape[:-1]) or p.shape[-1] % 4 or d.batch * d.M * d.N >= 2**31
+                or st.out_offset or st.out_dtype != dt.float32
+                or tuple(st.out_strides) != tuple(contiguous_strides(p.shape))):
+            continue
+        others = [w for s in plan.steps if s is not st and s is not d for w in list(s.inputs) + list(s.outputs)]
+        if any(buffer(w) == buffer(v) for w in others):
+            continue
+        cols = _swiglu_columns(p, v)
+        if cols is not None:
+            d.keep_planes = True
+            plan.steps[i] = SwigluPlanesStep(d, st, cols)
 
 
 def axis_view(shape, axis) -> Tuple[int, int, int]:

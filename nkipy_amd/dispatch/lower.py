@@ -272,6 +272,7 @@ class Lowering:
                 raise LoweringError(f"pattern {m} was never emitted")
         for res, outv in deferred:
             plan.steps.append(G.ProgramStep(f"write back {res.name}", G.flat_copy_program(res), outv))
+        G.fuse_swiglu_planes(plan)
         return plan
 
     _INPLACE_OPS = ("dynamic_update_slice", "scatter_along_axis", "put_along_axis", "scatter_strided")
