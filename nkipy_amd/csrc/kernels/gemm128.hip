@@ -33,7 +33,8 @@
 // x 4096 43.0 -> 36.9 us, K 14336, 128 x 4096 126 -> 102.  With two workgroups
 // per CU the four-wave form is the faster one (2000 x 4096 65 against 73).
 //
-// Few rows (_kh64, _kh32: at most 64 / 32 rows, one tile row): the same eight
+// Few rows (_kh64, _kh32; the first also for more rows while its tiles are at
+// most one per CU: 170 x 6144 x 4096 fp8 38 -> 28 us): the same eight
 // waves over 64 or 32 rows (2 or 1 MFMA row tiles per wave).  24 rows padded to
 // 128 leave the matrix pipes, not the weight stream, as the bound (0.55 us a
 // block, 15 KB/us a CU); the smaller tile and the deeper ring its A stage

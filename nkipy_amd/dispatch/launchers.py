@@ -295,7 +295,7 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
     (default: wherever it applies, i.e. 64-deep stages and a bf16 output in
     aligned 16-byte row chunks) writes the output tile through LDS so that
     every global store covers whole lines.  ``tile`` 128 selects the kernels
-    of 128 x 128 output tiles (gemm128.hip; no fp8 NN form, none of the other
+    of 128 x 128 output tiles, 64 those of 64 x 128 (gemm128.hip; no fp8 NN form, none of the other
     options), ``kh`` their eight-wave form (default: at most 256 tiles), 64 or
     32 its few-row form for that many rows (default: wherever M fits).
     """
@@ -335,11 +335,11 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
         raise LaunchError("SwiGLU with fp8 weights needs scales for both weights")
     if swiglu and (bias_ptr or resid_ptr or c_dtype != dt.bfloat16):
         raise LaunchError("the SwiGLU epilogue writes bf16 without bias / residual")
-    if tile not in (128, GEMM_BM):
-        raise LaunchError(f"GEMM output tiles are 128 or {GEMM_BM} wide, got {tile}")
-    if tile == 128 and ((fp8 and layout == "nn") or pingpong is not None or stage64 is not None or staged is not None):
+    if tile not in (64, 128, GEMM_BM):
+        raise LaunchError(f"GEMM output tiles have 64, 128 or {GEMM_BM} rows, got {tile}")
+    if tile <= 128 and ((fp8 and layout == "nn") or pingpong is not None or stage64 is not None or staged is not None):
         raise LaunchError("the 128-tile GEMM has no fp8 NN form and no kernel options")
-    bn = tile // 2 if swiglu else tile
+    bn = max(tile, 128) // (2 if swiglu else 1)
     tiles_m = -(-M // tile)
     tiles_n = -(-N // bn)
     if tiles_m * tiles_n >= 2**31:
@@ -383,11 +383,13 @@ def gemm(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, layout: 
     ctag = "bf16" if c_dtype == dt.bfloat16 else "f32"
     n_mm = 2 if swiglu else 1
     nbytes = M * K * 2 + n_mm * N * K * b_dtype.itemsize + M * N * c_dtype.itemsize
-    if tile == 128:
+    if tile <= 128:
+        if tile == 64 and kh not in (None, 64):
+            raise LaunchError("the 64-row GEMM tiles have the eight-wave form only")
         args.group_m = GEMM128_GROUP_M
         symbol = (f"nk_gemm128_swiglu_{layout}_{btag}_bf16" if swiglu else
                   f"nk_gemm128_{layout}_{btag}_{ctag}" + ("_rope" if rope is not None else ""))
-        kh = _gemm128_kh(kh, M, tiles_m * tiles_n)
+        kh = 64 if tile == 64 else _gemm128_kh(kh, M, tiles_m * tiles_n)
         symbol += f"_kh{kh or ''}" if kh is not None else ""
         return Launch("gemm128", symbol, (tiles_m * tiles_n, 1, 1), (256 if kh is None else 512, 1, 1), args,
                       bytes=nbytes, flops=2 * M * N * K * n_mm)
@@ -436,6 +438,11 @@ def _gemm128_kh(kh, M: int, workgroups: int):
     return kh
 
 
+# us per 1000 k of at most 256 workgroups of 64 x 128 tiles, beside _GEMM_US
+# (whose fixed part the model leaves out too)
+_GEMM64_US = {("nt", True): 4.6, ("nt", False): 6.3, ("nn", False): 7.4}
+
+
 REDUCE4_MIN = 1 << 17
 SPLITK_TARGET_WGS = 256  # one 8-wave GEMM workgroup per CU
 
@@ -479,7 +486,7 @@ GEMM128_MAX_RANGES = 16
 def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = False,
               ranges: bool = True) -> Tuple[int, int, int]:
     """(tile, K ranges, k per range) of the fastest GEMM form by the table
-    above: the 256 x 256 tiles where they fill whole rounds (4096 rows of a
+    above (tile 64: 64 x 128): the 256 x 256 tiles where they fill whole rounds (4096 rows of a
     12288-wide projection), the 128 x 128 tiles where the large ones leave CUs
     idle or padded (fp8, K 4096: 1000 x 6144 58 against 86 us, 1000 x 4096 37
     against 85), and those over K ranges where they still do (300 x 4096 x
@@ -501,7 +508,8 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
         if ks != want:
             continue
         # a SwiGLU pair in ranges runs as two launches, gate and up
-        wgs = -(-M // 128) * (-(-N // 64) if swiglu and ks == 1 else -(-N // 128)) * ks
+        tiles_n = -(-N // 64) if swiglu and ks == 1 else -(-N // 128)
+        wgs = -(-M // 128) * tiles_n * ks
         if M <= 64:
             rounds, few = -(-wgs // 256), n_mm if ks > 1 else 1
             weights = n_mm / few * N * K * (1 if fp8 else 2) / _GEMM_FEW_STREAM
@@ -511,6 +519,8 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
                 us += _GEMM_FEW_REDUCE + 8 * ks * M * N * n_mm / _PLANES_RATE
             best = min(best, (us, (128, ks, kc)))
             continue
+        if ks == 1 and -(-M // 64) * tiles_n <= 256:
+            best = min(best, (max(_GEMM64_US[(layout, fp8)] * K / 1000, stream), (64, 1, K)))
         us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
         if ks > 1:
             planes = 4 * ks * M * N * n_mm

@@ -110,15 +110,15 @@ def test_rotary_equals_the_256_tile_kernel(gpu, layout, bd):
     tx, tw, ts, tc, tsn = (_dev(a) for a in (dt.to_bf16(x), wd, scale, np.cos(ang).astype(np.float32),
                                              np.sin(ang).astype(np.float32)))
     got = []
-    for opt in ({}, {"tile": 128, "kh": False}, {"tile": 128, "kh": True}):
+    for opt in ({}, {"tile": 128, "kh": False}, {"tile": 128, "kh": True}, {"tile": 64}):
         q, k, c = (DeviceTensor.from_numpy(dt.to_bf16(np.zeros((M, n), np.float32))) for n in (nq, nk, Nn))
         rope = LA.GemmRope(tc.ptr, tsn.ptr, q.ptr, k.ptr, 64, S, nq, nk)
         LA.gemm(tx.ptr, tw.ptr, c.ptr, M, Nn, K, layout=layout, b_dtype=bd, c_dtype=dt.bfloat16,
                 scale_ptr=ts.ptr if ts else 0, rope=rope, **opt).run(gpu)
         gpu.sync()
         got.append([dt.to_float32(t.numpy()) for t in (q, k, c)])
-    for a, b, h in zip(*got):
-        assert np.array_equal(a, b)
+    for a, b, h, h64 in zip(*got):
+        assert np.array_equal(a, b) and np.array_equal(h, h64)
         # a product moved by one rounding step (2^-8 of it) moves both halves' rotations
         worst = float(np.max(np.abs(h - a)) / np.max(np.abs(a)))
         assert worst <= 2.0 ** -7
@@ -185,3 +185,29 @@ def test_few_row_tiles(gpu, M, Nn, K, layout, bd):
                 l.run(gpu)
             gpu.sync()
             _check(dt.to_float32(out.numpy()), ref, size)
+
+
+@pytest.mark.parametrize("layout,bd", FORMS)
+@pytest.mark.parametrize("M,Nn,K", [(65, 136, 80), (128, 264, 1056), (200, 128, 592), (321, 72, 640)])
+def test_64_row_tiles(gpu, layout, bd, M, Nn, K):
+    """Several 64-row tiles: plain with bias and residual, and as a SwiGLU
+    pair."""
+    print(f"gemm128 64-row tiles {layout} {dt.name(bd)} {M}x{Nn}x{K}", flush=True)
+    rng = np.random.default_rng(M + Nn + K)
+    x, w, wd, scale = _operands(rng, M, Nn, K, layout, bd)
+    _, u, ud, uscale = _operands(rng, M, Nn, K, layout, bd)
+    bias, resid = N.bf16_round(rng.standard_normal(Nn)), N.bf16_round(rng.standard_normal((M, Nn)))
+    tx, tw, ts, tu, tus, tb, tr = (_dev(a) for a in (dt.to_bf16(x), wd, scale, ud, uscale, dt.to_bf16(bias),
+                                                     dt.to_bf16(resid)))
+    g, v = (x.astype(np.float64) @ (m if layout == "nn" else m.T).astype(np.float64) for m in (w, u))
+    terms = np.abs(x).astype(np.float64) @ np.abs(w if layout == "nn" else w.T).astype(np.float64)
+    out = DeviceTensor.empty((M, Nn), dt.bfloat16)
+    kw = dict(layout=layout, b_dtype=bd, c_dtype=dt.bfloat16, scale_ptr=ts.ptr if ts else 0, tile=64)
+    l = LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, bias_ptr=tb.ptr, resid_ptr=tr.ptr, **kw)
+    assert l.symbol.endswith("_kh64") and l.grid[0] == -(-M // 64) * -(-Nn // 128)
+    l.run(gpu)
+    gpu.sync()
+    _check(dt.to_float32(out.numpy()), g + bias + resid, terms + 4)
+    LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, up_ptr=tu.ptr, up_scale_ptr=tus.ptr if tus else 0, **kw).run(gpu)
+    gpu.sync()
+    _check(dt.to_float32(out.numpy()), g / (1 + np.exp(-g)) * v, 8 * (1 + np.abs(g)) * (1 + np.abs(v)))
