@@ -1181,21 +1181,37 @@ def divide_rounds_as_multiply(div: float) -> bool:
         return bool(np.array_equal(dt.round_to_bf16(s / d), dt.round_to_bf16(s * (np.float32(1) / d))))
 
 
-def attention_stat_chunks(S: int, causal: bool = True):
+ATT_STAT_WGS = 512  # two workgroups per CU
+
+
+def attention_stat_chunks(S: int, causal: bool = True, heads: int = None):
     """Key chunks of the bf16 softmax's row statistics: (32-key blocks per
     chunk, most chunks of a query block, chunks summed over the query blocks
     of 128).  Chunks of 512 keys, or of S / 8 rounded up to 128 keys
-    when S passes 4096, so a row has at most 8."""
-    ckb = 4 * max(4, -(-S // 1024))
+    when S passes 4096, so a row has at most 8.  With fewer than two workgroups
+    per CU over ``heads`` (sequences x query heads) the chunks are halved, down
+    to 128 keys, while a row has at most 8.  Prefill layers, hidden 1024, 8
+    heads: 649 tokens 82 -> 70 us, 1800 141 -> 127; hidden 4096, 32 heads, 300
+    tokens 95 -> 90."""
     nb = -(-S // 32)
-    per_qb = [-(-(min((qb + 1) * 4, nb) if causal else nb) // ckb) for qb in range(-(-S // 128))]
-    return ckb, max(per_qb), sum(per_qb)
+
+    def split(ckb):
+        per_qb = [-(-(min((qb + 1) * 4, nb) if causal else nb) // ckb) for qb in range(-(-S // 128))]
+        return ckb, max(per_qb), sum(per_qb)
+
+    best = split(4 * max(4, -(-S // 1024)))
+    while heads and best[0] >= 8 and best[0] % 8 == 0 and heads * best[2] < ATT_STAT_WGS:
+        half = split(best[0] // 2)
+        if half[1] > 8:
+            break
+        best = half
+    return best
 
 
 def attention_rowstat_bytes(B: int, S: int, Hq: int, causal: bool = True) -> int:
     """Workspace of the bf16 softmax (ATT_SOFTMAX_BF16): per query and key
     chunk, the max score and the sum of the weights, as fp32."""
-    return 2 * 4 * attention_stat_chunks(S, causal)[1] * B * Hq * S
+    return 2 * 4 * attention_stat_chunks(S, causal, B * Hq)[1] * B * Hq * S
 
 
 def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq: int, Hkv: int,
@@ -1266,7 +1282,7 @@ def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq
         if score_flags & ATT_RND_SCORE and divide_rounds_as_multiply(float(div)):
             score_flags &= ~ATT_DIVIDE
             scale = float(np.float32(1) / div)
-    ckb, nch, items_per_head = attention_stat_chunks(S, causal) if smx_bf16 else (0, 0, 0)
+    ckb, nch, items_per_head = attention_stat_chunks(S, causal, B * Hq) if smx_bf16 else (0, 0, 0)
     args = AttnArgs(*vals, B, S, Hq, Hkv, float(scale), 1 if causal else 0, float(div),
                     float(np.float32(1.0) / np.float32(div)), int(score_flags), int(rowstat_ptr), ckb, nch)
     if score_flags:

@@ -1,5 +1,5 @@
-"""Routes of fp8 projections of few rows: the GEMM's few-row tiles, the MFMA
-few-row kernels, the VALU form."""
+"""Rules of the work splits: fp8 projections of few rows (the GEMM's few-row tiles, the MFMA
+few-row kernels, the VALU form), the row statistics of the bf16 softmax."""
 
 import pytest
 
@@ -28,3 +28,11 @@ def test_row_tiles_follow_the_rows(M, suffix):
     with pytest.raises(LA.LaunchError):
         LA.gemm(A, A, A, 65, 256, 256, layout="nt", b_dtype=dt.float8_e4m3fn, c_dtype=dt.bfloat16, scale_ptr=A,
                 tile=128, kh=64)
+
+
+@pytest.mark.parametrize("S,heads,want", [(24, 32, (4, 1, 1)), (649, 16, (4, 6, 21)), (1500, 32, (16, 3, 24)),
+                                          (1800, 8, (8, 8, 64)), (5000, 4, (20, 8, 180)), (5000, None, (20, 8, 180))])
+def test_row_statistics_chunks(S, heads, want):
+    assert LA.attention_stat_chunks(S, True, heads) == want
+    # whole query blocks of keys, so that no chunk starts past its queries
+    assert want[0] % 4 == 0 and want[1] <= 8
