@@ -85,6 +85,9 @@ _ROW_REG_VARIANTS = [(64, 1), (256, 1), (64, 8), (512, 4)]
 # every (block, chunks) pair compiled for the row kernels
 _ALL_REG_VARIANTS = {(64, 1), (128, 4), (256, 1), (256, 2), (512, 1), (256, 4), (512, 4)}
 _SOFTMAX_REG_VARIANTS = _ALL_REG_VARIANTS | {(64, 8)}
+# (block, elements per thread) of the element-wise register form, for rows not
+# in whole aligned 16-byte pieces, first fit; longer rows loop
+_SOFTMAX_ELT_VARIANTS = [(64, 4), (256, 4), (256, 8), (256, 16), (256, 32), (512, 32), (512, 64)]
 _SOFTMAX_TYPES = {("f32", "f32"), ("bf16", "bf16"), ("bf16", "f32"), ("f32", "bf16"), ("f16", "f16")}
 
 
@@ -122,6 +125,10 @@ def softmax_rows(x_ptr: int, y_ptr: int, rows: int, n: int, in_dtype, out_dtype,
     args = SoftmaxArgs(x_ptr, y_ptr, rows, n, SMX_ROUND_OPS if round_ops else 0)
     nbytes = rows * n * (dt.itemsize(in_dtype) + dt.itemsize(out_dtype))
     if var is None:
+        for block, per in _SOFTMAX_ELT_VARIANTS:
+            if n <= block * per:
+                return Launch("rowwise", f"nk_softmax_elt_{ti}_{to}_b{block}_e{per}", (rows, 1, 1), (block, 1, 1),
+                              args, bytes=nbytes)
         return Launch("rowwise", f"nk_softmax_loop_{ti}_{to}", (rows, 1, 1), (256, 1, 1),
                       args, bytes=nbytes, note="loop")
     block, chunks = var
