@@ -482,15 +482,16 @@ __device__ __forceinline__ void round_bf16x2(float &x0, float &x1) {
 // be partial: keys past S come in as zeros (past the end of the resources)
 // and are masked (causal: no stored query sees them), queries past S repeat
 // the last query's loads and store nothing.  The weights of the fp32 softmax
-// then enter the P V MFMAs as a pair of bf16 values, p = hi + lo to 2^-17
-// (two MFMAs per fragment): such lengths ran on the unfused kernels, whose
-// weights are fp32, and keep that accuracy.  Batch 2, S = 1000, 32 / 8 heads:
-// the fp8 attention block 6811 us unfused, 241 us with this kernel (and the
-// Qwen3 prefill layer of 1500 tokens 9387 -> 388 us).
+// then enter the P V MFMAs in three bf16 parts (three MFMAs per fragment),
+// each the leading eight bits of what is left of the weight, so that their
+// sum is the fp32 weight exactly: such lengths ran on the unfused kernels,
+// whose weights are fp32, and keep that precision.  Batch 2, S = 1000, 32 / 8
+// heads: the fp8 attention block 6811 us unfused, 231 us with this kernel (223
+// with the weights in two parts, 2^-17).
 template <int NW, bool XF = false, bool SMX = false, bool RAG = false>
 __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   static_assert(!SMX || XF, "the bf16 softmax follows the score cast points");
-  constexpr bool SPLIT = RAG && !SMX;  // weights as hi + lo
+  constexpr bool SPLIT = RAG && !SMX;  // weights in three bf16 parts
   constexpr int AQW = 32 * NW;  // queries per workgroup
   constexpr int TB = 32 * AD * 2;  // one 32-key K or V tile
   // one array per operand: a slot is a constant offset, so one address
@@ -633,9 +634,9 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s, 0, 0, 0);
     }
   };
-  // O^T += V^T P^T for one block (P as two 16-key bf16 fragments, SPLIT: and
-  // two of the rest of each weight)
-  constexpr int NP = SPLIT ? 4 : 2;
+  // O^T += V^T P^T for one block (P as two 16-key bf16 fragments, SPLIT: two
+  // of each part)
+  constexpr int NP = SPLIT ? 6 : 2;
   auto pv = [&](const uint8_t *Vt, const bf16x8_t (&pf)[NP]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -647,21 +648,40 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
           v[si] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(Vt + (16 * j + 8 * si) * 256 + voff(dt)));
         const bf16x8_t vf = __builtin_shufflevector(__builtin_bit_cast(bf16x4_t, v[0]),
                                                     __builtin_bit_cast(bf16x4_t, v[1]), 0, 1, 2, 3, 4, 5, 6, 7);
-        acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[j], acc_o[dt], 0, 0, 0);
-        if constexpr (SPLIT) acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[2 + j], acc_o[dt], 0, 0, 0);
+#pragma unroll
+        for (int part = 0; part < NP; part += 2)
+          acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[part + j], acc_o[dt], 0, 0, 0);
       }
   };
-  // p = 2^(s c - m) of one block -> bf16 fragments; returns this lane's sum
+  // p = 2^(s c - m) of one block -> bf16 fragments; returns this lane's sum.
+  // SPLIT: the parts of a weight are its fp32 bits cut after the leading
+  // eight significant ones, twice (p - hi and p - hi - mid are exact, and the
+  // last has at most eight)
   auto expblock = [&](const f32x16 &s, bf16x8_t (&pf)[NP]) __attribute__((always_inline)) {
     float ps0 = 0.f, ps1 = 0.f;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + e], sl2, -m_run));
-        if (e & 1) ps1 += p; else ps0 += p;
-        pf[j][e] = (__bf16)p;
-        if constexpr (SPLIT) pf[2 + j][e] = (__bf16)(p - (float)pf[j][e]);
+      for (int e = 0; e < 8; e += SPLIT ? 2 : 1) {
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + e], sl2, -m_run));
+        if constexpr (SPLIT) {
+          typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+          float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + e + 1], sl2, -m_run));
+          ps0 += p;
+          ps1 += p1;
+#pragma unroll
+          for (int part = 0; part < NP; part += 2) {
+            const uint32_t b0 = __float_as_uint(p), b1 = __float_as_uint(p1);
+            const bf16x2_t w = __builtin_bit_cast(bf16x2_t, __builtin_amdgcn_perm(b1, b0, 0x07060302u));
+            pf[part + j][e] = w[0];
+            pf[part + j][e + 1] = w[1];
+            p -= __uint_as_float(b0 & 0xffff0000u);
+            p1 -= __uint_as_float(b1 & 0xffff0000u);
+          }
+        } else {
+          if (e & 1) ps1 += p; else ps0 += p;
+          pf[j][e] = (__bf16)p;
+        }
       }
     return ps0 + ps1;
   };
@@ -743,7 +763,7 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
       __builtin_amdgcn_sched_group_barrier(0x100, 24, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
 #pragma unroll
-      for (int i = 0; i < (SPLIT ? 24 : 16); ++i) {
+      for (int i = 0; i < (SPLIT ? 32 : 16); ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
       }

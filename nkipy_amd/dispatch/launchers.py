@@ -1233,7 +1233,7 @@ def attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, B: int, S: int, Hq
     (4, 32), the last with three workgroups per CU; ``ring`` selects the
     software-pipelined (4, 32) kernel over a four-slot K / V ring.
     ``ragged`` selects that kernel's form for any S (partial last blocks of
-    queries and keys, the fp32 softmax's weights kept to 2^-17 as two bf16
+    queries and keys, the fp32 softmax's weights kept whole as three bf16
     parts); every other form needs S to be a multiple of 128.
 
     ``score_flags`` (ATT_*) give each score the traced code's cast points

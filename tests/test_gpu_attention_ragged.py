@@ -107,3 +107,39 @@ def test_lowering_takes_every_length(S):
     symbols = [l.symbol for p in (plan, bplan) for st in p.steps for l in st.launches(lambda v: 1 << 40)
                if "causal" in l.symbol]
     assert [("_rag" in s) for s in symbols] == [S % 128 != 0] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [35, 129, 353])
+def test_weights_keep_fp32(gpu, S):
+    """The weights of the fp32 softmax enter P V as fp32: value columns that
+    subtract a weight's leading 16 bits leave its last ones, which the bf16
+    output then shows.  Query 0's scores are 0 for three keys (p = 1) and -t
+    for a fourth; v sums to p - hi - mid with hi, mid the leading two groups
+    of eight bits of p = exp(-t)."""
+    rng = np.random.default_rng(S)
+    t = N.bf16_round(rng.uniform(0.05, 3, D)).astype(np.float64)
+    q = np.zeros((1, S, D, D))
+    k, v = np.zeros((1, S, 1, D)), np.zeros((1, S, 1, D))
+    keys = rng.permutation(S)[:4]
+    other = np.setdiff1d(np.arange(S), keys)
+    q[0, :, :, 0] = 2.0 ** 10  # every other key: a score of -2^15, weight 0
+    k[0, other, 0, 0] = -2.0 ** 5 * np.sqrt(D).astype(np.float32)
+    # head h: scores of the fourth key -t[h]
+    q[0, :, :, 1] = -t
+    k[0, keys[3], 0, 1] = 1.0
+    p = np.exp(-t / np.sqrt(D))
+    hi = N.bf16_round(p).astype(np.float64)
+    mid = N.bf16_round(p - hi).astype(np.float64)
+    # one column of v per head: the head's own column is read back
+    v[0, keys[0], 0], v[0, keys[1], 0], v[0, keys[3], 0] = -hi, -mid, 1.0
+    args = [N.bf16_round(a) for a in (q, k, v)]
+    assert np.array_equal(args[2], v)
+    got = _call(_unmasked, args, f"rag_weights_{S}").reshape(S, D, D)
+    left = np.array([got[:, h, h] for h in range(D)], np.float64) * (3 + p)[:, None]
+    # 2^-21 of the weight: its exponent's argument, the hardware's 2^x (1 ulp)
+    # and the fp32 sums, about 2^-24 each; the value subtracted to is at most
+    # 2^-18 of it, bf16 there is exact to 2^-26
+    worst = float(np.max(np.abs(left - (p - hi - mid)[:, None]) / p[:, None]))
+    print(f"weights to 2^{np.log2(worst):.1f}, left {np.max(np.abs(p - hi - mid)):.2e}", flush=True)
+    assert worst <= 2.0 ** -21
