@@ -486,7 +486,7 @@ __device__ __forceinline__ void round_bf16x2(float &x0, float &x1) {
 // each the leading eight bits of what is left of the weight, so that their
 // sum is the fp32 weight exactly: such lengths ran on the unfused kernels,
 // whose weights are fp32, and keep that precision.  Batch 2, S = 1000, 32 / 8
-// heads: the fp8 attention block 6811 us unfused, 231 us with this kernel (223
+// heads: the fp8 attention block 6811 us unfused, 236 us with this kernel (223
 // with the weights in two parts, 2^-17).
 template <int NW, bool XF = false, bool SMX = false, bool RAG = false>
 __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
@@ -656,7 +656,9 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
   // p = 2^(s c - m) of one block -> bf16 fragments; returns this lane's sum.
   // SPLIT: the parts of a weight are its fp32 bits cut after the leading
   // eight significant ones, twice (p - hi and p - hi - mid are exact, and the
-  // last has at most eight)
+  // last has at most eight).  No part of a weight is 0 (2^-126 instead, the
+  // least normal value, lost in any finite sum) so that an infinite v comes
+  // out infinite, as from the whole weight; a weight of 0 keeps its zeros
   auto expblock = [&](const f32x16 &s, bf16x8_t (&pf)[NP]) __attribute__((always_inline)) {
     float ps0 = 0.f, ps1 = 0.f;
 #pragma unroll
@@ -669,14 +671,15 @@ __device__ __forceinline__ void attention_sp_body(const AttnArgs &a) {
           float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * j + e + 1], sl2, -m_run));
           ps0 += p;
           ps1 += p1;
+          const float low0 = fminf(p, 0x1p-126f), low1 = fminf(p1, 0x1p-126f);
 #pragma unroll
           for (int part = 0; part < NP; part += 2) {
             const uint32_t b0 = __float_as_uint(p), b1 = __float_as_uint(p1);
             const bf16x2_t w = __builtin_bit_cast(bf16x2_t, __builtin_amdgcn_perm(b1, b0, 0x07060302u));
             pf[part + j][e] = w[0];
             pf[part + j][e + 1] = w[1];
-            p -= __uint_as_float(b0 & 0xffff0000u);
-            p1 -= __uint_as_float(b1 & 0xffff0000u);
+            p = fmaxf(p - __uint_as_float(b0 & 0xffff0000u), low0);
+            p1 = fmaxf(p1 - __uint_as_float(b1 & 0xffff0000u), low1);
           }
         } else {
           if (e & 1) ps1 += p; else ps0 += p;

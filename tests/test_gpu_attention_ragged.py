@@ -143,3 +143,17 @@ def test_weights_keep_fp32(gpu, S):
     worst = float(np.max(np.abs(left - (p - hi - mid)[:, None]) / p[:, None]))
     print(f"weights to 2^{np.log2(worst):.1f}, left {np.max(np.abs(p - hi - mid)):.2e}", flush=True)
     assert worst <= 2.0 ** -21
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [True, False])
+def test_infinite_values(gpu, causal):
+    """An infinite v comes out infinite in every query that sees its key, in
+    its column alone."""
+    S, at = 200, 70
+    q, k, v = _qkv(1, S, 2, 1)
+    v[0, at, 0, 5], v[0, at, 0, 9] = np.inf, -np.inf
+    got = _call(causal_gqa_attention_kernel if causal else _unmasked, (q, k, v), f"rag_inf_{causal}")
+    sees = got.reshape(1, S, 2, D)[0, at if causal else 0:]
+    assert np.all(sees[..., 5] == np.inf) and np.all(sees[..., 9] == -np.inf)
+    assert np.all(np.isfinite(np.delete(sees, [5, 9], axis=-1)))
