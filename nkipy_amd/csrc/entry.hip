@@ -187,13 +187,15 @@ int nkh_linear_attention(const void *q, const void *k, const void *v, void *o, i
   rc = check_ptrs(q, k, v, o);
   if (rc) return rc;
   const size_t need = (size_t)least_workspace(bh, t);
-  const LinAttnSplit split = linattn_split_within(bh, t, workspace ? workspace_size : 0);
+  // (an unaligned workspace holds no split: one that is not needed may be any pointer)
+  const bool aligned = reinterpret_cast<uintptr_t>(workspace) % 16 == 0;
+  const LinAttnSplit split = linattn_split_within(bh, t, workspace && aligned ? workspace_size : 0);
   if (need && (!workspace || workspace_size < need))
     return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention of BH=" + std::to_string(bh) + " T=" +
                                                         std::to_string(t) + " needs a workspace of " +
                                                         std::to_string(need) + " bytes, got " +
                                                         std::to_string(workspace_size));
-  if (split.nranges && reinterpret_cast<uintptr_t>(workspace) % 16)
+  if (need && !aligned)
     return nkh_internal::set_error(NKH_ERR_INVALID, "linear attention workspace must be 16-byte aligned");
   return nkh_internal::with_stream([&](hipStream_t stream, int) {
     return launch_linattn(q, k, v, o, bh, t, split, static_cast<float *>(workspace), stream);

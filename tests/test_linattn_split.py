@@ -1,6 +1,8 @@
 """The linear-attention work split: segments and ranges cover the chunks, one
 workgroup per CU, never dearer than the long segments by its own time model."""
 
+import ctypes
+
 import pytest
 
 from nkipy_amd.dispatch import launchers as LA
@@ -17,3 +19,25 @@ def test_split_covers_the_sequence(bh, chunks):
     cost = LA._linattn_cost(bh, chunks, nseg, rchunks)
     assert (nseg, rchunks) == long or cost < LA._linattn_cost(bh, chunks, *long)
     assert LA.linear_attention_workspace_bytes(bh, 64 * chunks) >= bh * nranges * 129 * 128 * 4
+
+
+def test_c_abi_ignores_a_workspace_it_does_not_need():
+    """A shape that needs no workspace takes any pointer as one: the shorter
+    segments use it only where it is aligned and large enough.  Without a
+    device the call passes its checks and stops at the missing runtime."""
+    from nkipy_amd.runtime.hip import load_library
+
+    lib = load_library()
+    flag = ctypes.c_int()
+    assert lib.nkh_is_initialized(ctypes.byref(flag)) == 0
+    if flag.value:
+        pytest.skip("the call would launch")
+    bh, t, size = 24, 768, ctypes.c_size_t()
+    assert LA._linattn_long_split(bh, t)[0] == 1 and LA.linear_attention_split(bh, t)[0] > 1
+    assert lib.nkh_linear_attention_workspace_size(bh, t, ctypes.byref(size)) == 0
+    p = 1 << 20
+    codes = {lib.nkh_linear_attention(p, p, p, p, bh, t, ws, n)
+             for ws, n in ((None, 0), (p, size.value), (p + 8, size.value), (p + 8, 16))}
+    assert codes == {lib.nkh_linear_attention(p, p, p, p, bh, 64, None, 0)}
+    # one that needs a workspace wants it aligned
+    assert lib.nkh_linear_attention(p, p, p, p, 1, 4096, p + 8, 1 << 30) == 2
