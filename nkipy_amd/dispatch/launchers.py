@@ -1094,7 +1094,8 @@ def linear_attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, BH: int, T:
     Returns the launches in order: when the sequences are cut into segments,
     a partial-sum kernel writes the prefix states into ``part_ptr`` (a
     workspace of :func:`linear_attention_workspace_bytes` bytes) before the
-    scan reads them.  With ``vmax_ptr`` (BH uint32 words) the scan writes
+    scan reads them; without one the long segments are taken, where
+    those need none.  With ``vmax_ptr`` (BH uint32 words) the scan writes
     each sequence's max |v| as bf16 bits there, for
     :func:`check_linear_attention_vmax` after the launches complete."""
     if (D, Dv, chunk) != (LINATTN_D, LINATTN_D, LINATTN_CHUNK):
@@ -1105,6 +1106,9 @@ def linear_attention(q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, BH: int, T:
     if any(p % 16 for p in (q_ptr, k_ptr, v_ptr, o_ptr)):
         raise LaunchError("linear attention operands must be 16-byte aligned")
     nseg, rchunks, nranges = linear_attention_split(BH, T, ranges_per_segment)
+    if nranges and not part_ptr:
+        nseg, rchunks = _linattn_long_split(BH, T, ranges_per_segment)
+        nranges = (nseg - 1) * (T // chunk // nseg // rchunks)
     if BH * nseg >= 2**31 or BH * max(nranges, 1) >= 2**31:
         raise LaunchError("linear attention grid too large")
     if nranges and not part_ptr:

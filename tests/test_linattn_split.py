@@ -41,3 +41,14 @@ def test_c_abi_ignores_a_workspace_it_does_not_need():
     assert codes == {lib.nkh_linear_attention(p, p, p, p, bh, 64, None, 0)}
     # one that needs a workspace wants it aligned
     assert lib.nkh_linear_attention(p, p, p, p, 1, 4096, p + 8, 1 << 30) == 2
+
+
+def test_launcher_without_a_workspace():
+    """The launcher needs a workspace only where the long segments do; without
+    one the sequences run unsegmented."""
+    p = 1 << 20
+    plain = LA.linear_attention(p, p, p, p, 24, 768)
+    assert [l.symbol for l in plain] == ["nk_linattn_c64_d128"] and plain[0].args.nseg == 1
+    assert len(LA.linear_attention(p, p, p, p, 24, 768, part_ptr=p)) == 2
+    with pytest.raises(LA.LaunchError):
+        LA.linear_attention(p, p, p, p, 1, 4096)
