@@ -618,11 +618,12 @@ def _reduce_planes(args: "GemvArgs", c_dtype, swiglu: bool) -> Launch:
     """The launch that adds a projection's partial planes and applies the
     epilogue: one wave per four ranges over 64 outputs, or, from
     ``REDUCE4_MIN`` outputs on, four outputs per thread (24 x 4096 from 8
-    planes 4.8 us either way, 64 x 6144 from 5 planes 9.1 against 5.0)."""
+    planes 4.8 us either way, 64 x 6144 from 5 planes 9.1 against 5.0), whose
+    32-bit indices end at 2^31 outputs."""
     out = GemvArgs.from_buffer_copy(args)
     plane = out.M * out.N
     vb = 4 * c_dtype.itemsize
-    four = (plane >= REDUCE4_MIN and out.N % 4 == 0 and out.ldc % 4 == 0 and out.C % vb == 0
+    four = (REDUCE4_MIN <= plane < 2**31 and out.N % 4 == 0 and out.ldc % 4 == 0 and out.C % vb == 0
             and (not out.resid or out.resid % vb == 0))
     if four:
         out.flags |= GEMV_OUT4

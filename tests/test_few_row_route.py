@@ -36,3 +36,14 @@ def test_row_statistics_chunks(S, heads, want):
     assert LA.attention_stat_chunks(S, True, heads) == want
     # whole query blocks of keys, so that no chunk starts past its queries
     assert want[0] % 4 == 0 and want[1] <= 8
+
+
+@pytest.mark.parametrize("M,N,four", [(1 << 10, 1 << 7, True), (1 << 10, 127, False), ((1 << 15) - 1, 1 << 16, True),
+                                      (1 << 15, 1 << 16, False), (1 << 16, (1 << 16) + 8, False)])
+def test_reduction_of_large_outputs_keeps_64_bit_indices(M, N, four):
+    """The form of four outputs per thread indexes rows and columns in 32
+    bits: outputs of 2^31 elements and more take the other one."""
+    out = LA.gemm_splitk(A, A, A, M, N, 128, layout="nt", b_dtype=dt.bfloat16, c_dtype=dt.bfloat16, ws_ptr=A,
+                         split=(2, 64))[-1]
+    assert out.symbol == "nk_gemv_out_bf16" and bool(out.args.flags & LA.GEMV_OUT4) is four
+    assert out.grid[0] == -(-M * N // (1024 if four else 64))
