@@ -535,6 +535,8 @@ class HeadRopePattern:
                 st = [vv.simple(d) for d in range(4)]
                 if any(v is None for v in st) or st[3] != 1:
                     continue
+                if vv.offset % 8 or any(v % 8 for v in st[:3]):  # the launch copies 16-byte pieces
+                    continue
                 out = [dict(m) for m in ms]
                 out[i].update(out=kw["out"], o_str=kw["o_str"], o_pos=kw["o_pos"], o_off=kw.get("o_off", 0),
                               nodes=km["nodes"] + [kw["node"]])
