@@ -194,6 +194,18 @@ def copy16(src_ptr: int, dst_ptr: int, nbytes: int) -> Launch:
                   Copy16Args(src_ptr, dst_ptr, n16, grid * 256), bytes=2 * nbytes)
 
 
+def copy_words(src_ptr: int, dst_ptr: int, nbytes: int) -> Launch:
+    """Device copy of 16-bit elements at any address (a one-load program)."""
+    total = nbytes // 2
+    grid = _grid_for(total)
+    a = EwArgs()
+    a.out, a.total, a.rank, a.n_in, a.n_instr, a.nthreads = dst_ptr, total, 1, 1, 1, grid * 256
+    a.shape[0], a.out_strides[0], a.out_dtype = total, 1, dtype_code(dt.uint16)
+    a.inp[0].ptr, a.inp[0].strides[0], a.inp[0].dtype = src_ptr, 1, dtype_code(dt.uint16)
+    a.prog[0].op, a.prog[0].dtype = OP_LOAD, dtype_code(dt.uint16)
+    return Launch("generic", "nk_ew_program", (grid, 1, 1), (256, 1, 1), a, bytes=2 * nbytes)
+
+
 class DecodeE4m3Args(ctypes.Structure):
     _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("n8", ctypes.c_int64),
                 ("nthreads", ctypes.c_int64)]

@@ -241,7 +241,10 @@ class HeadRopeMatch(Match):
         desc = f"head rope B={B} S={S} D={D} bf16 steps: " + ", ".join(parts) + \
             (" (runtime position)" if tb["pos"] is not None else "") + \
             (f" from {planes[1]} partial-sum planes" if planes else "")
-        return [LaunchStep("head_rope", desc, self.inputs, self.outputs, make)]
+        step = LaunchStep("head_rope", desc, self.inputs, self.outputs, make)
+        # (caches written at a fixed offset: a program takes them at any address)
+        step.any_address = tuple(m["out"] for m in members if m.get("o_pos") == (0, 0))
+        return [step]
 
 
 class HeadRopePattern:
@@ -826,7 +829,10 @@ class AttentionMatch(Match):
             desc += f" keys<{S} of {self.keys}"
         if self.score_flags:
             desc += f" score_flags={self.score_flags}"
-        return [LaunchStep("attention", desc, self.inputs, self.outputs, make)]
+        step = LaunchStep("attention", desc, self.inputs, self.outputs, make)
+        if S % 128:  # (the unfused kernels of such lengths take any address)
+            step.any_address = (q.base, k.base, v.base, out)
+        return [step]
 
 
 def _qk_dot(n: Node) -> bool:

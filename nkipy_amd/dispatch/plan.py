@@ -19,13 +19,13 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass, field
-from typing import Callable, Dict, List, Optional
+from typing import Callable, Dict, List, Optional, Tuple
 
 import numpy as np
 
 from nkipy_amd.core import dtypes as dt
 from nkipy_amd.core.backend.ir import Graph, Value
-from nkipy_amd.dispatch.launchers import Launch
+from nkipy_amd.dispatch.launchers import Launch, LaunchError
 
 
 @dataclass
@@ -47,6 +47,10 @@ class Step:
     """One lowered unit of work: one or more kernel launches."""
 
     kind = "step"
+    # operands whose launches want 16-byte alignment but whose caller may hold
+    # them anywhere: an argument buffer of theirs at another address goes
+    # through an aligned copy (PlanExecutor)
+    any_address: Tuple[Value, ...] = ()
 
     def __init__(self, desc: str, inputs: List[Value], outputs: List[Value]):
         self.desc = desc
@@ -241,6 +245,7 @@ class PlanExecutor:
         self._full: Optional[Plan] = plan if isinstance(plan, Plan) else None
         self.rt = get_runtime()
         self._owned: Dict[int, DeviceBuffer] = {}
+        self._copies: Dict[tuple, DeviceBuffer] = {}  # aligned copies of argument buffers, by their indices
         pname = plan.graph.name if isinstance(plan, Plan) else plan.name
         for b in plan.buffers:
             if b.kind in ("temp", "const"):
@@ -271,16 +276,54 @@ class PlanExecutor:
                 + list(self.plan.output_buffers.values())):
             return self.plan.bind(bases, self.rt)
         plan = self._full_plan()
+        before: List[Launch] = []
+        after: List[Launch] = []
 
         def addr(v) -> int:
             # a graph value, or a Slot of a step's own workspace temporary
             s = v if isinstance(v, Slot) else plan.slot(v)
             return bases[s.buffer] + s.offset
 
-        launches: List[Launch] = []
-        for st in plan.steps:
-            launches.extend(st.launches(addr))
-        return BoundPlan(launches, self.rt)
+        def refused(st) -> bool:
+            try:
+                st.launches(addr)
+            except LaunchError:
+                return True
+            return False
+
+        if any(bases[i] % 16 for i in list(plan.input_buffers.values()) + list(plan.output_buffers.values())):
+            moved = [plan.slot(v).buffer for st in plan.steps if st.any_address and refused(st)
+                     for v in st.any_address]
+            bases, before, after = self._aligned_copies(plan, bases, moved)
+        launches = [l for st in plan.steps for l in st.launches(addr)]
+        return BoundPlan(before + launches + after, self.rt)
+
+    def _aligned_copies(self, plan: Plan, bases: Dict[int, int], moved: List[int]):
+        """Copies of the argument buffers ``moved`` that are not 16-byte
+        aligned, for the duration of an execution: (addresses with those of
+        the copies, launches that fill them, launches that write results
+        back).  An output shares the copy of the input it aliases.  The copies
+        are kept as the temporaries are, the same ones for every binding."""
+        from nkipy_amd.dispatch.generic import copy_words
+        from nkipy_amd.runtime.device_tensor import DeviceBuffer
+
+        bases, before, after = dict(bases), [], []
+        for ptr in dict.fromkeys(bases[i] for i in moved if plan.buffers[i].kind in ("input", "output")):
+            if ptr % 16 == 0:
+                continue
+            group = [b for b in plan.buffers if b.kind in ("input", "output") and bases[b.index] == ptr]
+            nbytes = max(b.nbytes for b in group)
+            key = tuple(b.index for b in group)
+            buf = self._copies.get(key)
+            if buf is None:
+                buf = self._copies[key] = DeviceBuffer(max(nbytes, 16), name=f"{plan.graph.name}:aligned{key[0]}")
+            if any(b.kind == "input" for b in group):
+                before.append(copy_words(ptr, buf.ptr, nbytes))
+            if any(b.kind == "output" for b in group):
+                after.append(copy_words(buf.ptr, ptr, nbytes))
+            for b in group:
+                bases[b.index] = buf.ptr
+        return bases, before, after
 
     def bind(self, io_ptrs: Dict[str, int]) -> BoundPlan:
         """``io_ptrs``: input / output name -> device address."""
@@ -332,11 +375,13 @@ class PlanExecutor:
         """Drop every bound launch list and owned buffer without touching the
         device (the runtime they belong to is gone)."""
         self._owned.clear()
+        self._copies.clear()
         self._bound.clear()
 
     def close(self):
         self._release_graphs()
-        for b in self._owned.values():
+        for b in list(self._owned.values()) + list(self._copies.values()):
             b.free()
         self._owned.clear()
+        self._copies.clear()
         self._bound.clear()
