@@ -308,11 +308,24 @@ struct EwfArgs {
 };
 typedef float f32v16 __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ float ewf_load1(const void *p, int32_t i, int dt) {
-  if (dt == DT_F32) return ((const float *)p)[i];
-  if (dt == DT_BF16) return bf16_to_f32(((const uint16_t *)p)[i]);
-  if (dt == DT_F16) return f16_to_f32(((const uint16_t *)p)[i]);
-  return ((const uint8_t *)p)[i] ? 1.f : 0.f;
+// four elements at offsets o: all loads in flight before the first is widened
+__device__ __forceinline__ void ewf_gather(const void *p, const int32_t (&o)[4], int dt, float (&v)[4]) {
+  if (dt == DT_F32) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = ((const float *)p)[o[e]];
+  } else if (dt == DT_BOOL) {
+    uint8_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = ((const uint8_t *)p)[o[e]];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = h[e] ? 1.f : 0.f;
+  } else {
+    uint16_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = ((const uint16_t *)p)[o[e]];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = dt == DT_BF16 ? bf16_to_f32(h[e]) : f16_to_f32(h[e]);
+  }
 }
 __device__ __forceinline__ float ewf_round(float v, int dt) {
   if (dt == DT_BF16) return bf16_to_f32(f32_to_bf16(v));
@@ -378,13 +391,14 @@ extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) {
               }
             } else {
               const int32_t s = in.strides[a.rank - 1];  // 0: broadcast
-#pragma unroll
-              for (int e = 0; e < 4; ++e) v[e] = ewf_load1(in.ptr, o + e * s, in.dtype);
+              const int32_t at[4] = {o, o + s, o + 2 * s, o + 3 * s};
+              ewf_gather(in.ptr, at, in.dtype, v);
             }
           } else {
+            int32_t at[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              v[e] = ewf_load1(in.ptr, offset(in.strides, lin + min((uint32_t)e, n - 1)), in.dtype);
+            for (int e = 0; e < 4; ++e) at[e] = offset(in.strides, lin + min((uint32_t)e, n - 1));
+            ewf_gather(in.ptr, at, in.dtype, v);
           }
           break;
         }

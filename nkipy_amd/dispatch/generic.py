@@ -124,6 +124,7 @@ _EWF_OPS = {OP_LOAD, OP_CONST, OP_SELECT} | set(COMPARE_CODES.values()) | {
                              "round_nearest_even", "trunc", "sign", "is_finite", "is_nan", "logistic", "copy")} | {
     BINARY_CODES[n] for n in ("add", "subtract", "multiply", "divide", "maximum", "minimum")}
 _EWF_NOT = UNARY_CODES["not"]
+EWF_RAGGED_MIN = 512 * 256  # a round of nk_ew_program: two workgroups per CU
 
 
 def collapse_dims(shape, strides):
@@ -481,6 +482,13 @@ class ProgramStep(Step):
         shape, strides = collapse_dims(p.shape, [self.out_strides] + [s for _, s, _ in p.inputs])
         span = max(sum(abs(st) * (n - 1) for n, st in zip(shape, ss)) for ss in strides)
         if span >= 2**31:
+            return None
+        # rows that are no multiple of four cost a thread four index
+        # decompositions an operand: no gain before the general kernel's one
+        # element per thread fills more than one round (us there / here: an
+        # added row over 1000 x 33 9.0 / 9.9, four operands 11.0 / 12.0, a
+        # transpose of 33 x 2 x 5 x 64 8.4 / 10.0; 4001 x 33 12.5 / 9.9)
+        if len(shape) > 1 and shape[-1] % 4 and total <= EWF_RAGGED_MIN:
             return None
 
         def mode(ptr, st, isz):

@@ -88,3 +88,34 @@ def test_collapse_dims():
     # a transpose merges nothing; size-1 dimensions go
     assert G.collapse_dims((3, 1, 4), [full((3, 1, 4)), [1, 7, 3]]) == ([3, 4], [[4, 1], [1, 3]])
     assert G.collapse_dims((1, 1), [[1, 1]]) == ([1], [[0]])
+
+
+def _ragged(x, y, z):
+    t = np.transpose(y)
+    m = np.greater(x, t)
+    return x + t * z, np.where(m, np.flip(x, axis=0), z), m, np.flip(t, axis=x.ndim - 1) - x
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(5, 3, 2), (7, 1, 3), (2, 3, 2, 3, 3), (3, 2, 2, 3, 2, 3), (9, 5), (130, 1001)])
+@pytest.mark.parametrize("d", ["float32", "float16", "bfloat16"])
+def test_ragged_rows_equal_the_general_kernel(gpu, monkeypatch, shape, d):
+    """Innermost dimensions shorter than, or no multiple of, a thread's four
+    elements, at the sizes that the rule leaves to the general kernel too:
+    reversed, transposed and broadcast operands, a mask."""
+    print(f"elementwise ragged {shape} {d}", flush=True)
+    monkeypatch.setattr(G, "EWF_RAGGED_MIN", -1)
+    rng = np.random.default_rng(len(shape))
+    arrays = [rng.standard_normal(s).astype(np.float32) for s in (shape, shape[::-1], shape[-1:])]
+    res, symbols = _both(_ragged, [dt.to_bf16(x) if d == "bfloat16" else x.astype(d) for x in arrays], monkeypatch)
+    assert symbols[0] == {"nk_ew_f32"} and "nk_ew_f32" not in symbols[1]
+    assert res[0] == res[1]
+
+
+@pytest.mark.parametrize("shape,symbol", [((1000, 33), "nk_ew_program"), ((1000, 32), "nk_ew_f32"),
+                                          ((3971, 33), "nk_ew_program"), ((3972, 33), "nk_ew_f32"),
+                                          ((1, 33), "nk_ew_f32")])
+def test_small_ragged_programs_take_the_general_kernel(shape, symbol):
+    x, row = np.zeros(shape, np.float32), np.zeros(shape[-1:], np.float32)
+    plan = lower(NKIPyKernel.trace(lambda x, y: x + y).specialize(x, row))
+    assert [l.symbol for st in plan.steps for l in st.launches(lambda v: 1 << 40)] == [symbol]
