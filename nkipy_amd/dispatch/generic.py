@@ -648,10 +648,27 @@ def _dot_span(esz: int, s_row: int, s_k: int, rows: int, K: int) -> int:
     return ((max(rows, 1) - 1) * s_row + (max(K, 1) - 1) * s_k + 1) * esz
 
 
+def dot_small(batch: int, M: int, N: int, K: int, half: bool, scalar: bool) -> bool:
+    """Whether an unsplit product stays on nk_dot's 16 x 16 tiles: where the
+    matrix-core tiles are mostly padding, or where the product ends within a
+    few steps and nk_dot's shorter prologue wins (``half``: a 16-bit operand,
+    ``scalar``: one loaded element by element).  us, nk_dot / nk_dot_f32:
+    8192 of 16 x 16 x 16 11.7 / 30.7, 8192 of 17 x 17 x 4 34.5 / 40.4 (but of
+    32 x 64 x 16 68.6 / 37.8); bf16 64 x 64 x 64 6.7 / 8.1, 512 of 16 x 200 x 8
+    10.7 / 13.8, 512 of 33 x 33 x 17 11.3 / 8.6; fp32 16 of 33 x 33 x 33
+    6.4 / 8.1, 128 of 33 x 33 x 33 7.7 / 8.2, 512 of 33 x 33 x 8 8.8 / 8.2,
+    64 of 64 x 64 x 64 (vector loads) 8.2 / 6.9."""
+    tiles = -(-M // 16) * -(-N // 16)
+    steps = batch * tiles * -(-K // 16)
+    if tiles == 1 or (tiles <= 4 and max(M, N) <= 64 and K <= 16):
+        return True
+    return (K <= 256 and steps <= 7168) if half else (scalar and K <= 128 and steps <= 3456)
+
+
 class DotStep(Step):
     """Fallback batched dot with arbitrary operand strides (fp32 accumulate):
     fp32, fp16 and bf16 operands on the matrix cores (nk_dot_f32), other
-    types on nk_dot."""
+    types and small products (:func:`dot_small`) on nk_dot."""
 
     kind = "dot"
 
@@ -698,7 +715,13 @@ class DotStep(Step):
         self.split, self.planes = (1, self.K), None
         self.keep_planes = False  # the consumer adds them (SwigluPlanesStep)
         outputs = self.batch * self.M * self.N
-        self.tile = dot_tile(self.M, self.N, a_v.dtype == dt.float32 and b_v.dtype == dt.float32)
+        pair32 = a_v.dtype == dt.float32 and b_v.dtype == dt.float32
+        self.tile = dot_tile(self.M, self.N, pair32)
+        if self.f32 and outputs > 0:
+            ranges = dot_split(self.batch, self.M, self.N, self.K, self.tile)[0] if node.out.dtype != dt.float16 else 1
+            scalar = 0 in (_dot_mode(0, 1, self.sam, self.sak, self.sab, self.M, self.K, self.batch),
+                           _dot_mode(0, 1, self.sbn, self.sbk, self.sbb, self.N, self.K, self.batch))
+            self.f32 = ranges > 1 or not dot_small(self.batch, self.M, self.N, self.K, not pair32, scalar)
         if self.f32 and plan is not None and outputs > 0:
             # (the reduction writes fp32 or bf16)
             ks, kc = dot_split(self.batch, self.M, self.N, self.K, self.tile)
@@ -839,7 +862,7 @@ def fuse_swiglu_planes(plan):
             continue
         v = st.prog.inputs[0][0]
         dots = [d for d in plan.steps[:i] if isinstance(d, DotStep) and d.node.out.id == v.id]
-        if len(dots) != 1 or not dots[0].f32 or v.dtype != dt.float32 or buffer(v) is None:
+        if len(dots) != 1 or v.dtype != dt.float32 or buffer(v) is None:
             continue
         d, p = dots[0], st.prog
         if (plan.buffers[buffer(v)].kind != "temp" or d.N != v.shape[-1] or d.N % 4 or len(p.shape) != v.ndim

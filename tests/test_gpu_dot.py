@@ -7,8 +7,10 @@ import numpy as np
 import pytest
 
 from nkipy_amd.core import dtypes as dt
+from nkipy_amd.core.trace import NKIPyKernel
 from nkipy_amd.dispatch import generic as G
-from nkipy_amd.runtime import baremetal_jit
+from nkipy_amd.dispatch.lower import lower
+from nkipy_amd.runtime import DeviceKernel, DeviceTensor, baremetal_jit
 
 
 def _nn(a, b):
@@ -105,3 +107,37 @@ def test_tile_choice():
     assert all(G.dot_tile(M, N, True) == (32, 128) for _, M, N, _ in WIDE)
     assert G.dot_tile(2, 1024, False) == (64, 64) and G.dot_tile(1, 64, True) == (64, 64)
     assert G.dot_tile(33, 4096, True) == (64, 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("batch,M,N,K", sorted(set(SIZES + WIDE)))
+@pytest.mark.parametrize("types", [("float32", "float32"), ("float16", "float32"), ("float32", "bfloat16")])
+def test_matrix_core_form_at_small_sizes(gpu, monkeypatch, form, batch, M, N, K, types):
+    """nk_dot_f32 at the sizes that dot_small leaves to nk_dot: the same edges
+    of tiles, stages and load modes."""
+    monkeypatch.setattr(G, "dot_small", lambda *a: False)
+    monkeypatch.setitem(globals(), "baremetal_jit", _uncached)
+    test_products_match_float64(gpu, form, batch, M, N, K, types)
+
+
+def _uncached(fn):
+    def call(*args):
+        dk = DeviceKernel.compile_and_load(fn, *args, name="dot_small_off", use_cached_if_exists=False)
+        symbols = [l.symbol for st in dk.plan.steps for l in st.launches(lambda v: 1 << 40)]
+        assert "nk_dot" not in symbols or fn is FORMS["reversed"][0]
+        ins = {n: DeviceTensor.from_numpy(a, name=n) for n, a in zip(dk.input_tensors_info, args)}
+        return dk(ins)["output0"].numpy()
+    return call
+
+
+@pytest.mark.parametrize("batch,M,N,K,d,symbol", [
+    (4096, 16, 16, 16, "float32", "nk_dot"), (1, 16, 16, 8192, "float32", "nk_dot_f32_f1_f2"),
+    (4096, 17, 17, 4, "float32", "nk_dot"), (4096, 32, 64, 64, "float32", "nk_dot_f32_f1_f2"),
+    (1, 64, 64, 64, "float16", "nk_dot"), (1, 64, 64, 64, "float32", "nk_dot_f32_f1_f2"),
+    (1, 33, 33, 33, "float32", "nk_dot"), (512, 33, 33, 33, "float32", "nk_dot_f32_f0_f0"),
+    (512, 33, 33, 17, "float16", "nk_dot_f32_h0_h0"), (1, 64, 64, 512, "float16", "nk_dot_f32_h1_h2"),
+    (1, 8, 8, 0, "float32", "nk_dot")])
+def test_small_products_keep_the_small_tiles(batch, M, N, K, d, symbol):
+    plan = lower(NKIPyKernel.trace(_nn).specialize(np.zeros((batch, M, K), d), np.zeros((batch, K, N), d)))
+    assert plan.steps[0].launches(lambda v: 1 << 40)[0].symbol == symbol
