@@ -507,6 +507,8 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
     stream = n_mm * N * K * (1 if fp8 else 2) / _GEMM_STREAM
     tiles256 = -(-M // 256) * -(-(N * n_mm) // 256)
     best = (max(stream, -(-tiles256 // 256) * c256 * K / 1000), (GEMM_BM, 1, K))
+    if M <= 64:  # (the few-row times hold the fixed part, the others leave it out)
+        best = best[0] + _GEMM_FIXED_US, best[1]
     if M > GEMM128_MAX_M:
         return best[1]
     for want in range(1, (GEMM128_MAX_RANGES if ranges else 1) + 1):
