@@ -485,6 +485,15 @@ _GEMM_FEW_US = {("nt", True): 4.9, ("nt", False): 6.5, ("nn", False): 6.4}
 _GEMM_FIXED_US = 6.0      # launch, prologue, epilogue
 _GEMM_STREAM = 4.5e6      # weight bytes per us a short product streams at
 _PLANES_RATE = 5.0e6      # partial-sum bytes per us, written and read again
+# a bf16 SwiGLU pair of 2^24 weights and more in rounds of the four-wave form,
+# beside _GEMM_US: its 64 columns of each weight a tile read half lines (198
+# rows of 2 x 14336 x 4096 94 us, 83 on the 256 x 256 tiles; 1237 of 2 x 7168 x
+# 5120 251 / 238, but 1269 of 2 x 3072 x 2048 0.80 of them)
+_GEMM_PAIR_COST, _GEMM_PAIR_WEIGHTS = 1.25, 1 << 24
+# past 64 rows the 128-tile forms are taken where the times above say 5% less
+# (2049 rows of 4096 x 14336 bf16 NT in three ranges: a tie by them, 364 against
+# 284 us with the weights in cache)
+_GEMM128_GAIN = 0.95
 GEMM128_MAX_M = 8192      # rows past which the 256 x 256 tiles fill the part at every width in use
 GEMM128_MAX_RANGES = 16
 
@@ -507,8 +516,8 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
     stream = n_mm * N * K * (1 if fp8 else 2) / _GEMM_STREAM
     tiles256 = -(-M // 256) * -(-(N * n_mm) // 256)
     best = (max(stream, -(-tiles256 // 256) * c256 * K / 1000), (GEMM_BM, 1, K))
-    if M <= 64:  # (the few-row times hold the fixed part, the others leave it out)
-        best = best[0] + _GEMM_FIXED_US, best[1]
+    # (the few-row times hold the fixed part, the others leave it out)
+    best = (best[0] + _GEMM_FIXED_US if M <= 64 else best[0] * _GEMM128_GAIN, best[1])
     if M > GEMM128_MAX_M:
         return best[1]
     for want in range(1, (GEMM128_MAX_RANGES if ranges else 1) + 1):
@@ -531,6 +540,8 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
         if ks == 1 and -(-M // 64) * tiles_n <= 256:
             best = min(best, (max(_GEMM64_US[(layout, fp8)] * K / 1000, stream), (64, 1, K)))
         us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
+        if swiglu and not fp8 and ks == 1 and wgs > 256 and N * K >= _GEMM_PAIR_WEIGHTS:
+            us *= _GEMM_PAIR_COST
         if ks > 1:
             planes = 4 * ks * M * N * n_mm
             if planes > 1 << 28:
