@@ -498,6 +498,17 @@ GEMM128_MAX_M = 8192      # rows past which the 256 x 256 tiles fill the part at
 GEMM128_MAX_RANGES = 16
 
 
+def _gemm_few_us(M: int, N: int, K: int, layout: str, fp8: bool, n_mm: int, ks: int, kc: int) -> float:
+    """Time of the few-row form (at most 64 rows) by the table above."""
+    # a SwiGLU pair in ranges runs as two launches, gate and up
+    wgs = (-(-N // 64) if n_mm > 1 and ks == 1 else -(-N // 128)) * ks
+    rounds, few = -(-wgs // 256), n_mm if ks > 1 else 1
+    weights = n_mm / few * N * K * (1 if fp8 else 2) / _GEMM_FEW_STREAM
+    us = few * (rounds * _GEMM_FEW_ROUND + (
+        weights ** 3 + (rounds * _GEMM_FEW_US[(layout, fp8)] * kc / 1000) ** 3) ** (1 / 3))
+    return us + (_GEMM_FEW_REDUCE + 8 * ks * M * N * n_mm / _PLANES_RATE if ks > 1 else 0)
+
+
 @functools.lru_cache(maxsize=4096)
 def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = False,
               ranges: bool = True) -> Tuple[int, int, int]:
@@ -525,18 +536,12 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
         ks = -(-K // kc)
         if ks != want:
             continue
+        if M <= 64:
+            best = min(best, (_gemm_few_us(M, N, K, layout, fp8, n_mm, ks, kc), (128, ks, kc)))
+            continue
         # a SwiGLU pair in ranges runs as two launches, gate and up
         tiles_n = -(-N // 64) if swiglu and ks == 1 else -(-N // 128)
         wgs = -(-M // 128) * tiles_n * ks
-        if M <= 64:
-            rounds, few = -(-wgs // 256), n_mm if ks > 1 else 1
-            weights = n_mm / few * N * K * (1 if fp8 else 2) / _GEMM_FEW_STREAM
-            us = few * (rounds * _GEMM_FEW_ROUND + (
-                weights ** 3 + (rounds * _GEMM_FEW_US[(layout, fp8)] * kc / 1000) ** 3) ** (1 / 3))
-            if ks > 1:
-                us += _GEMM_FEW_REDUCE + 8 * ks * M * N * n_mm / _PLANES_RATE
-            best = min(best, (us, (128, ks, kc)))
-            continue
         if ks == 1 and -(-M // 64) * tiles_n <= 256:
             best = min(best, (max(_GEMM64_US[(layout, fp8)] * K / 1000, stream), (64, 1, K)))
         us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
@@ -797,20 +802,43 @@ def gemv_mfma_preferred(M: int, N: int, K: int, swiglu: bool = False, layout: st
     return M <= GEMV_MFMA_MAX_M and tiles * -(-K // 256) <= _GEMV_MFMA_TARGET_WGS
 
 
+# the fp8 NT form's time, us: fixed (two launches), per MB of weights, per MB of
+# planes, per round of 256 k and 16 rows (cold weights, 2 to 32 rows, 4 k to 157 M
+# weights: within 20%)
+_GEMV_MFMA_US = (8.8, 0.19, 0.21, 1.2)
+_GEMM_FEW_GAIN = 0.95
+
+
+def _gemv_mfma_us(M: int, N: int, K: int, swiglu: bool) -> float:
+    n_mm = 2 if swiglu else 1
+    ks, kc = gemv_mfma_split(M, N, K, swiglu)
+    rounds = -(-(-(-N // (128 if swiglu else 256)) * ks) // _GEMV_MFMA_TARGET_WGS)
+    fixed, weights, planes, step = _GEMV_MFMA_US
+    return (fixed + weights * n_mm * N * K / 1e6 + planes * 8 * ks * M * N * n_mm / 1e6
+            + step * -(-M // 16) * rounds * kc / 256)
+
+
 def gemm_few_preferred(M: int, N: int, K: int, swiglu: bool = False, layout: str = "nn",
                        fp8: bool = False) -> bool:
     """Whether the GEMM's few-row tiles are the form for fp8 NT weights that
     :func:`gemv_mfma_preferred` or :func:`gemv_preferred` take too (measured with
-    cold weights): a SwiGLU pair whose 64-column tiles reach 48 of the CUs in one
-    K loop without planes (12 rows of 2 x 14336 x 4096 27.5 against 39.3 us, 2 x
-    3072 x 1024 10.0 against 11.4; but 2 x 1536 x 2048, 24 tiles, 14.8 against
-    10.7); plain, 17 rows and more (24 of 6144 x 4096 15.4 against 20.2, of 2048
-    x 1536 10.5 against 12.2), fewer from 2^25 weights on (12 of 4096 x 14336
+    cold weights): a SwiGLU pair whose 64-column tiles reach 48 of the CUs, where
+    the two forms' modelled times say so (12 rows of 2 x 14336 x 4096 29.0 against
+    41.2 us, 2 x 3072 x 1024 11.8 against 12.8; but 2 x 4096 x 4096, a long K loop
+    on 64 CUs or ranges in two launches, 24.8 against 18.6, and 2 x 1536 x 2048,
+    24 tiles, 14.8 against 10.7); plain, 17 rows and more (24 of 6144 x 4096
+    15.4 against 20.2, of 2048 x 1536 10.5 against 12.2), fewer from 2^25 weights on (12 of 4096 x 14336
     21.3 against 23.4; of 4096 x 4096 13.1 against 11.9).  One row streams
     faster on the VALU form."""
     if M <= 1 or layout != "nt" or not fp8:
         return False
-    return -(-N // 64) >= 48 if swiglu else M > 16 or N * K >= 1 << 25
+    if not swiglu:
+        return M > 16 or N * K >= 1 << 25
+    if -(-N // 64) < 48 or not gemv_mfma_preferred(M, N, K, True, layout, fp8):
+        return -(-N // 64) >= 48
+    tile, ks, kc = gemm_form(M, N, K, layout, fp8, True)
+    return tile == 128 and (_gemm_few_us(M, N, K, layout, fp8, 2, ks, kc)
+                            <= _GEMM_FEW_GAIN * _gemv_mfma_us(M, N, K, True))
 
 
 def gemv_mfma_workspace_bytes(M: int, N: int, K: int, swiglu: bool = False) -> int:

@@ -47,3 +47,13 @@ def test_reduction_of_large_outputs_keeps_64_bit_indices(M, N, four):
                          split=(2, 64))[-1]
     assert out.symbol == "nk_gemv_out_bf16" and bool(out.args.flags & LA.GEMV_OUT4) is four
     assert out.grid[0] == -(-M * N // (1024 if four else 64))
+
+
+@pytest.mark.parametrize("M,N,K,want", [(2, 4096, 4096, False), (32, 4096, 4096, False), (2, 3072, 2048, False),
+                                        (16, 4096, 8192, False), (24, 4096, 8192, True), (4, 6144, 4096, False),
+                                        (8, 12288, 4096, True), (2, 14336, 4096, True), (16, 6144, 2048, True),
+                                        (8, 3072, 1024, True), (48, 4096, 4096, True)])
+def test_few_row_tiles_of_a_pair_follow_the_models(M, N, K, want):
+    """A SwiGLU pair whose K loop is long for its tiles, or runs in ranges,
+    stays on the MFMA few-row kernels."""
+    assert LA.gemm_few_preferred(M, N, K, True, "nt", True) is want
