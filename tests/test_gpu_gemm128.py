@@ -34,6 +34,13 @@ def _dev(a):
     return DeviceTensor.from_numpy(a) if a is not None else None
 
 
+def _clear(*tensors):
+    """NaN everywhere, so that a launch under test has to write every element
+    (and, in a workspace, every element that it reads)."""
+    for t in tensors:
+        t.write_from_numpy(np.full(t.nbytes, 0xff, np.uint8).view(t.dtype).reshape(t.shape))
+
+
 def _check(got, ref, terms, rounded=0.0):
     # bf16 rounding of the result and of a value `rounded` on the way (each at
     # most 2^-8 of it) and fp32 sums whose terms' sizes add up to `terms`
@@ -55,6 +62,7 @@ def test_plain_bias_residual_and_ranges(gpu, M, Nn, K, layout, bd, kh):
     terms = np.abs(x).astype(np.float64) @ np.abs(w if layout == "nn" else w.T).astype(np.float64)
     out = DeviceTensor.empty((M, Nn), dt.bfloat16)
     kw = dict(layout=layout, b_dtype=bd, c_dtype=dt.bfloat16, scale_ptr=ts.ptr if ts else 0, kh=kh)
+    _clear(out)
     LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, tile=128, bias_ptr=tb.ptr, resid_ptr=tr.ptr, **kw).run(gpu)
     gpu.sync()
     _check(dt.to_float32(out.numpy()), prod + bias + resid, terms + 4)
@@ -62,6 +70,7 @@ def test_plain_bias_residual_and_ranges(gpu, M, Nn, K, layout, bd, kh):
     kc = -(-(-(-K // ks)) // 64) * 64
     ks = -(-K // kc)
     ws = DeviceTensor.empty((ks, M, Nn), np.float32)
+    _clear(out, ws)
     for l in LA.gemm_splitk(tx.ptr, tw.ptr, out.ptr, M, Nn, K, split=(ks, kc), ws_ptr=ws.ptr,
                             resid_ptr=tr.ptr, round_before_resid=True, **kw):
         l.run(gpu)
@@ -83,12 +92,14 @@ def test_swiglu(gpu, M, Nn, K, layout, bd, kh):
     out = DeviceTensor.empty((M, Nn), dt.bfloat16)
     kw = dict(layout=layout, b_dtype=bd, c_dtype=dt.bfloat16, scale_ptr=ts.ptr if ts else 0, up_ptr=tu.ptr,
               up_scale_ptr=tus.ptr if tus else 0, kh=kh)
+    _clear(out)
     LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, tile=128, **kw).run(gpu)
     gpu.sync()
     _check(dt.to_float32(out.numpy()), ref, 8 * (1 + np.abs(g)) * (1 + np.abs(v)))
     kc = -(-(-(-K // 2)) // 64) * 64
     ks = -(-K // kc)
     ws = DeviceTensor.empty((2, ks, M, Nn), np.float32)
+    _clear(out, ws)
     for l in LA.gemm_splitk(tx.ptr, tw.ptr, out.ptr, M, Nn, K, split=(ks, kc), ws_ptr=ws.ptr, **kw):
         l.run(gpu)
     gpu.sync()
@@ -131,10 +142,11 @@ def test_reduction_forms_agree(gpu, ks, c_dtype):
     the same order: the same bits, plain, biased and with a residual."""
     M, Nn = 37, 264
     rng = np.random.default_rng(ks)
-    planes = DeviceTensor.from_numpy(rng.standard_normal((2, ks, M, Nn), dtype=np.float32))
-    scale = DeviceTensor.from_numpy(rng.uniform(0.5, 2, Nn).astype(np.float32))
-    bias = DeviceTensor.from_numpy(dt.to_bf16(rng.standard_normal(Nn).astype(np.float32)))
+    pl = rng.standard_normal((2, ks, M, Nn), dtype=np.float32)
+    sc, bi = rng.uniform(0.5, 2, Nn).astype(np.float32), N.bf16_round(rng.standard_normal(Nn))
+    planes, scale, bias = (DeviceTensor.from_numpy(a) for a in (pl, sc, dt.to_bf16(bi)))
     r = rng.standard_normal((M, Nn)).astype(np.float32)
+    r = N.bf16_round(r) if c_dtype == dt.bfloat16 else r
     resid = DeviceTensor.from_numpy(dt.to_bf16(r) if c_dtype == dt.bfloat16 else r)
     out = DeviceTensor.empty((M, Nn), c_dtype)
     flags = LA.GEMM_BIAS | LA.GEMM_SCALE | LA.GEMM_RESID | LA.GEMM_RND_BIAS | LA.GEMM_RND_RESID
@@ -147,12 +159,32 @@ def test_reduction_forms_agree(gpu, ks, c_dtype):
         for least in (1 << 62, 0):
             saved, LA.REDUCE4_MIN = LA.REDUCE4_MIN, least
             try:
-                LA._reduce_planes(args, c_dtype, swiglu).run(gpu)
+                l = LA._reduce_planes(args, c_dtype, swiglu)
             finally:
                 LA.REDUCE4_MIN = saved
+            assert bool(l.args.flags & LA.GEMV_OUT4) is (least == 0)
+            _clear(out)
+            l.run(gpu)
             gpu.sync()
             got.append(out.numpy().tobytes())
         assert got[0] == got[1]
+        # fp32 sums of ks terms; the rounding of the result and, with the
+        # epilogue, of the product and the biased product to bf16
+        g, u = pl.astype(np.float64).sum(1)
+        sums = 2.0 ** -22 * np.abs(pl).astype(np.float64).sum(1).max(0)
+        last = 2.0 ** -8 if c_dtype == dt.bfloat16 else 2.0 ** -23
+        if swiglu:
+            ref = g * sc / (1 + np.exp(-g * sc)) * (u * sc)
+            bound = last * np.abs(ref) + 8 * sums * (1 + np.abs(g)) * (1 + np.abs(u)) * sc * sc
+        elif fl:
+            p, b = g * sc, g * sc + bi
+            ref = b + r
+            bound = last * np.abs(ref) + 2.0 ** -8 * (np.abs(p) + np.abs(b)) + 4 * sums * sc
+        else:
+            ref, bound = g, last * np.abs(g) + sums
+        o = out.numpy()
+        o = dt.to_float32(o) if c_dtype == dt.bfloat16 else o
+        assert np.all(np.abs(o - ref) <= bound + 1e-30)
 
 
 @pytest.mark.parametrize("layout,bd", FORMS)
@@ -178,9 +210,11 @@ def test_few_row_tiles(gpu, M, Nn, K, layout, bd):
         for opt, ref, size in ((kw, g, terms), (pair, g / (1 + np.exp(-g)) * v, 8 * (1 + np.abs(g)) * (1 + np.abs(v)))):
             l = LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, tile=128, **opt)
             assert l.symbol.endswith(f"_kh{kh}")
+            _clear(out)
             l.run(gpu)
             gpu.sync()
             _check(dt.to_float32(out.numpy()), ref, size)
+            _clear(out, ws)
             for l in LA.gemm_splitk(tx.ptr, tw.ptr, out.ptr, M, Nn, K, split=(ks, kc), ws_ptr=ws.ptr, **opt):
                 l.run(gpu)
             gpu.sync()
@@ -205,9 +239,11 @@ def test_64_row_tiles(gpu, layout, bd, M, Nn, K):
     kw = dict(layout=layout, b_dtype=bd, c_dtype=dt.bfloat16, scale_ptr=ts.ptr if ts else 0, tile=64)
     l = LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, bias_ptr=tb.ptr, resid_ptr=tr.ptr, **kw)
     assert l.symbol.endswith("_kh64") and l.grid[0] == -(-M // 64) * -(-Nn // 128)
+    _clear(out)
     l.run(gpu)
     gpu.sync()
     _check(dt.to_float32(out.numpy()), g + bias + resid, terms + 4)
+    _clear(out)
     LA.gemm(tx.ptr, tw.ptr, out.ptr, M, Nn, K, up_ptr=tu.ptr, up_scale_ptr=tus.ptr if tus else 0, **kw).run(gpu)
     gpu.sync()
     _check(dt.to_float32(out.numpy()), g / (1 + np.exp(-g)) * v, 8 * (1 + np.abs(g)) * (1 + np.abs(v)))
