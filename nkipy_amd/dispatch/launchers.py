@@ -270,7 +270,6 @@ GEMM_RND_RESID = 32
 GEMM_ROWS16 = 64
 GEMV_OUT4 = 128
 GEMM_BM = 256
-GEMM_BN = 256
 GEMM128_GROUP_M = 8  # tile rows per group of the 128-tile kernels' walk
 
 
@@ -451,25 +450,6 @@ _GEMM64_US = {("nt", True): 4.6, ("nt", False): 6.3, ("nn", False): 7.4}
 
 
 REDUCE4_MIN = 1 << 17
-SPLITK_TARGET_WGS = 256  # one 8-wave GEMM workgroup per CU
-
-
-def gemm_splitk_split(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = False):
-    """(ksplit, kc) for :func:`gemm_splitk`: K ranges of kc (a multiple of
-    64) so that tiles x ranges is about one workgroup per CU.  Past 64 rows
-    each range's fp32 partial plane (4 M N bytes, written once and read once)
-    costs as much as its share of the K loop saves, so the planes are held
-    to half the weight bytes (measured at 4096 x 4096: 256 rows in 16 ranges
-    66 us against 80 us in one loop, 128 rows in 8 ranges 42 us); ksplit 1
-    when the tiles alone fill the part."""
-    tiles = -(-M // GEMM_BM) * -(-N // GEMM_BN)
-    ks = max(1, min(SPLITK_TARGET_WGS // tiles, -(-K // 64)))
-    if M > 64:
-        ks = max(1, min(ks, (N * K * (1 if fp8 else 2)) // (2 * 4 * M * N)))
-    kc = -(-(-(-K // ks)) // 64) * 64
-    return -(-K // kc), kc
-
-
 # Times of the GEMM forms, us per 1000 k of a round of workgroups (measured
 # cold, 24 to 3000 rows of 4096 / 6144 / 12288 / 14336-wide projections): a
 # round of 256 workgroups of 256 x 256 tiles; at most 256 workgroups of 128 x
@@ -485,10 +465,10 @@ _GEMM_FEW_US = {("nt", True): 4.9, ("nt", False): 6.5, ("nn", False): 6.4}
 _GEMM_FIXED_US = 6.0      # launch, prologue, epilogue
 _GEMM_STREAM = 4.5e6      # weight bytes per us a short product streams at
 _PLANES_RATE = 5.0e6      # partial-sum bytes per us, written and read again
-# a bf16 SwiGLU pair of 2^24 weights and more in rounds of the four-wave form,
-# beside _GEMM_US: its 64 columns of each weight a tile read half lines (198
-# rows of 2 x 14336 x 4096 94 us, 83 on the 256 x 256 tiles; 1237 of 2 x 7168 x
-# 5120 251 / 238, but 1269 of 2 x 3072 x 2048 0.80 of them)
+# a bf16 SwiGLU pair of 2^24 weights and more in rounds of the four-wave form
+# costs up to that much more than _GEMM_US says (measured, the cause is not
+# known: 198 rows of 2 x 14336 x 4096 94 us, 83 on the 256 x 256 tiles; 1237 of
+# 2 x 7168 x 5120 251 / 238; but 1269 of 2 x 3072 x 2048 0.80 of their time)
 _GEMM_PAIR_COST, _GEMM_PAIR_WEIGHTS = 1.25, 1 << 24
 # past 64 rows the 128-tile forms are taken where the times above say 5% less
 # (2049 rows of 4096 x 14336 bf16 NT in three ranges: a tie by them, 364 against
@@ -509,6 +489,36 @@ def _gemm_few_us(M: int, N: int, K: int, layout: str, fp8: bool, n_mm: int, ks: 
     return us + (_GEMM_FEW_REDUCE + 8 * ks * M * N * n_mm / _PLANES_RATE if ks > 1 else 0)
 
 
+def _gemm128_forms(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool, ranges: bool):
+    """(us, (tile, K ranges, k per range)) of the 128-column forms by the
+    tables above; ``ranges`` False: one K loop per tile."""
+    _, ckh, c128 = _GEMM_US[(layout, fp8)]
+    n_mm = 2 if swiglu else 1
+    stream = n_mm * N * K * (1 if fp8 else 2) / _GEMM_STREAM
+    for want in range(1, (GEMM128_MAX_RANGES if ranges else 1) + 1):
+        kc = -(-(-(-K // want)) // 64) * 64
+        ks = -(-K // kc)
+        if ks != want:
+            continue
+        if M <= 64:
+            yield _gemm_few_us(M, N, K, layout, fp8, n_mm, ks, kc), (128, ks, kc)
+            continue
+        # a SwiGLU pair in ranges runs as two launches, gate and up
+        tiles_n = -(-N // 64) if swiglu and ks == 1 else -(-N // 128)
+        wgs = -(-M // 128) * tiles_n * ks
+        if ks == 1 and -(-M // 64) * tiles_n <= 256:
+            yield max(_GEMM64_US[(layout, fp8)] * K / 1000, stream), (64, 1, K)
+        us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
+        if swiglu and not fp8 and ks == 1 and wgs > 256 and N * K >= _GEMM_PAIR_WEIGHTS:
+            us *= _GEMM_PAIR_COST
+        if ks > 1:
+            planes = 4 * ks * M * N * n_mm
+            if planes > 1 << 28:
+                continue
+            us = n_mm * (max(us, stream / n_mm) + _GEMM_FIXED_US) + 2 * planes / _PLANES_RATE
+        yield max(us, stream), (128, ks, kc)
+
+
 @functools.lru_cache(maxsize=4096)
 def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = False,
               ranges: bool = True) -> Tuple[int, int, int]:
@@ -522,38 +532,22 @@ def gemm_form(M: int, N: int, K: int, layout: str, fp8: bool, swiglu: bool = Fal
     read once, and a second launch.  ``ranges`` False: one K loop per tile."""
     if fp8 and layout == "nn":
         return GEMM_BM, 1, K
-    c256, ckh, c128 = _GEMM_US[(layout, fp8)]
     n_mm = 2 if swiglu else 1
     stream = n_mm * N * K * (1 if fp8 else 2) / _GEMM_STREAM
     tiles256 = -(-M // 256) * -(-(N * n_mm) // 256)
-    best = (max(stream, -(-tiles256 // 256) * c256 * K / 1000), (GEMM_BM, 1, K))
+    us = max(stream, -(-tiles256 // 256) * _GEMM_US[(layout, fp8)][0] * K / 1000)
     # (the few-row times hold the fixed part, the others leave it out)
-    best = (best[0] + _GEMM_FIXED_US if M <= 64 else best[0] * _GEMM128_GAIN, best[1])
+    best = (us + _GEMM_FIXED_US if M <= 64 else us * _GEMM128_GAIN, (GEMM_BM, 1, K))
     if M > GEMM128_MAX_M:
         return best[1]
-    for want in range(1, (GEMM128_MAX_RANGES if ranges else 1) + 1):
-        kc = -(-(-(-K // want)) // 64) * 64
-        ks = -(-K // kc)
-        if ks != want:
-            continue
-        if M <= 64:
-            best = min(best, (_gemm_few_us(M, N, K, layout, fp8, n_mm, ks, kc), (128, ks, kc)))
-            continue
-        # a SwiGLU pair in ranges runs as two launches, gate and up
-        tiles_n = -(-N // 64) if swiglu and ks == 1 else -(-N // 128)
-        wgs = -(-M // 128) * tiles_n * ks
-        if ks == 1 and -(-M // 64) * tiles_n <= 256:
-            best = min(best, (max(_GEMM64_US[(layout, fp8)] * K / 1000, stream), (64, 1, K)))
-        us = (ckh if wgs <= 256 else -(-wgs // 256) / 2 * c128) * kc / 1000
-        if swiglu and not fp8 and ks == 1 and wgs > 256 and N * K >= _GEMM_PAIR_WEIGHTS:
-            us *= _GEMM_PAIR_COST
-        if ks > 1:
-            planes = 4 * ks * M * N * n_mm
-            if planes > 1 << 28:
-                continue
-            us = n_mm * (max(us, stream / n_mm) + _GEMM_FIXED_US) + 2 * planes / _PLANES_RATE
-        best = min(best, (max(us, stream), (128, ks, kc)))
-    return best[1]
+    return min([best, *_gemm128_forms(M, N, K, layout, fp8, swiglu, ranges)])[1]
+
+
+def gemm_splitk_split(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = False) -> Tuple[int, int]:
+    """(K ranges, k per range) that :func:`gemm_splitk` takes by itself: the
+    fastest by the tables of :func:`gemm_form` (bf16 weights: those of NT)."""
+    forms = [f for f in _gemm128_forms(M, N, K, "nt", fp8, swiglu, True) if f[1][0] == 128]
+    return min(forms)[1][1:]
 
 
 def gemm_splitk_workspace_bytes(M: int, N: int, K: int, swiglu: bool = False, fp8: bool = False) -> int:
@@ -566,8 +560,9 @@ def gemm_splitk(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int, K: int, *, l
                 scale_ptr: int = 0, resid_ptr: int = 0, up_ptr: int = 0, up_scale_ptr: int = 0,
                 round_before_bias: bool = False, round_before_resid: bool = False,
                 split: Tuple[int, int] = None, kh: bool = None) -> List[Launch]:
-    """The operation of :func:`gemm` (no rotary form) for few rows: the
-    128-tile kernels over K ranges (grid y) into fp32 partial planes in the workspace
+    """The operation of :func:`gemm` (no rotary form) for products whose tiles
+    leave CUs idle: the 128-tile kernels over K ranges (grid y) into fp32
+    partial planes in the workspace
     at ``ws_ptr`` (``gemm_splitk_workspace_bytes``; the SwiGLU form runs the
     gate and the up weights into two sets of planes), then the reduction of
     :func:`gemv` adds the ranges in order and applies the epilogue.  bf16 NN,
