@@ -278,11 +278,12 @@ extern "C" __global__ __launch_bounds__(256) void nk_ew_program(EwArgs a) {
 // fp32, each instruction is decoded once for four consecutive elements of the
 // innermost dimension, inputs contiguous there load as one vector, and the
 // dimensions come collapsed from the host (usually one or two).  The results
-// are the other kernel's bit for bit: an fp32 sum, difference, product or
-// quotient equals the double one rounded to fp32 (53 >= 2 * 24 + 2 bits), and
-// the transcendental functions are evaluated in double here too.  That program,
-// a SiLU with its product over 200 x 3072 fp32: 38 us there, 9.4 us here (0.8
-// TB/s; the double exp of each element bounds it).
+// are the other kernel's bit for bit: an fp32 sum, difference, product, quotient
+// or root equals the double one rounded to fp32 (53 >= 2 * 24 + 2 bits; and 24
+// >= 2 * 11 + 2 for fp16 by way of fp32), and the transcendental functions are
+// evaluated in double here too and narrowed in one rounding (ewf_narrow).
+// That program, a SiLU with its product over 200 x 3072 fp32: 38 us there, 9.4
+// us here (0.8 TB/s; the double exp of each element bounds it).
 // ---------------------------------------------------------------------------
 #define EWF_MAX_RANK 6
 struct EwfInput {
@@ -333,6 +334,30 @@ __device__ __forceinline__ float ewf_round(float v, int dt) {
   if (dt == DT_BOOL) return v != 0.f ? 1.f : 0.f;
   return v;
 }
+// A double result as the fp32 that ewf_round narrows.  nk_ew_program's double
+// reaches fp16 in one rounding (the compiler contracts its two conversions); on
+// the way to fp16 this one is rounded to odd (toward zero, an inexact one with
+// its last bit set), which keeps the fp16 rounding from seeing a tie that the
+// double is not on: exp(0.02269) lies 2.7e-8 below the middle of two fp16
+// values and its nearest fp32 is that middle.  bf16 results are the same either
+// way, for every operand of that type.
+template <bool F16FN>
+__device__ __forceinline__ float ewf_narrow(double d, int dt) {
+  if (F16FN) {
+    // fp32 keeps the upper 23 of 52 fraction bits: the 29 below become one (by
+    // a mask: a branch on dt spills registers)
+    const uint32_t m = dt == DT_F16 ? 0x1fffffffu : 0u;
+    const uint64_t u = (uint64_t)__double_as_longlong(d);
+    const uint32_t lo = (uint32_t)u;
+    const uint32_t odd = (lo | ((lo & m) + m)) & ~m;
+    d = __longlong_as_double((long long)((u & 0xffffffff00000000ull) | odd));
+  }
+  const float f = (float)d;
+  // one element's function at a time: interleaved, the four need 37 registers
+  // more than there are at four waves per SIMD
+  if (F16FN) __builtin_amdgcn_sched_barrier(0);
+  return f;
+}
 __device__ __forceinline__ void ewf_store1(void *p, int32_t i, int dt, float v) {
   if (dt == DT_F32) ((float *)p)[i] = v;
   else if (dt == DT_BF16) ((uint16_t *)p)[i] = f32_to_bf16(v);
@@ -340,7 +365,12 @@ __device__ __forceinline__ void ewf_store1(void *p, int32_t i, int dt, float v) 
   else ((uint8_t *)p)[i] = v != 0.f ? 1 : 0;
 }
 
-extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) {
+// F16FN: some function's result is fp16.  A kernel of its own, so that the other
+// programs' code stays without the mask and the barriers.  The SiLU program
+// above in fp16 over 4096 x 4096, a call: 175 us, 163..178 us without the
+// narrowing, 1065 us in nk_ew_program (200 x 3072: 30 / 30 / 64 us).
+template <bool F16FN>
+__device__ __forceinline__ void ewf_body(const EwfArgs &a) {
   for (uint64_t lin0 = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4; lin0 < a.total; lin0 += a.step) {
     const uint32_t lin = (uint32_t)lin0;
     const uint32_t n = min(4u, a.total - lin);
@@ -405,11 +435,11 @@ extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) {
         EWF(OP_CONST, I.imm)
         EWF(OP_NEG, -x[e])
         EWF(OP_ABS, fabsf(x[e]))
-        EWF(OP_EXP, (float)exp((double)x[e]))
-        EWF(OP_LOG, (float)log((double)x[e]))
+        EWF(OP_EXP, ewf_narrow<F16FN>(exp((double)x[e]), I.dtype))
+        EWF(OP_LOG, ewf_narrow<F16FN>(log((double)x[e]), I.dtype))
         EWF(OP_SQRT, (float)sqrt((double)x[e]))
-        EWF(OP_RSQRT, (float)(1.0 / sqrt((double)x[e])))
-        EWF(OP_TANH, (float)tanh((double)x[e]))
+        EWF(OP_RSQRT, ewf_narrow<F16FN>(1.0 / sqrt((double)x[e]), I.dtype))
+        EWF(OP_TANH, ewf_narrow<F16FN>(tanh((double)x[e]), I.dtype))
         EWF(OP_CEIL, ceilf(x[e]))
         EWF(OP_FLOOR, floorf(x[e]))
         EWF(OP_RINT, rintf(x[e]))
@@ -417,7 +447,7 @@ extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) {
         EWF(OP_SIGN, (x[e] > 0.f) ? 1.f : ((x[e] < 0.f) ? -1.f : x[e]))
         EWF(OP_ISFINITE, isfinite(x[e]) ? 1.f : 0.f)
         EWF(OP_ISNAN, isnan(x[e]) ? 1.f : 0.f)
-        EWF(OP_LOGISTIC, (float)(1.0 / (1.0 + exp(-(double)x[e]))))
+        EWF(OP_LOGISTIC, ewf_narrow<F16FN>(1.0 / (1.0 + exp(-(double)x[e])), I.dtype))
         EWF(OP_COPY, x[e])
         EWF(OP_ADD, x[e] + y[e])
         EWF(OP_SUB, x[e] - y[e])
@@ -464,6 +494,9 @@ extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) {
     }
   }
 }
+
+extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32(EwfArgs a) { ewf_body<false>(a); }
+extern "C" __global__ __launch_bounds__(256, 4) void nk_ew_f32_f16fn(EwfArgs a) { ewf_body<true>(a); }
 
 // ---------------------------------------------------------------------------
 // SwiGLU over a fp32 product's partial planes: with P the sum of the planes in

@@ -124,6 +124,9 @@ _EWF_OPS = {OP_LOAD, OP_CONST, OP_SELECT} | set(COMPARE_CODES.values()) | {
                              "round_nearest_even", "trunc", "sign", "is_finite", "is_nan", "logistic", "copy")} | {
     BINARY_CODES[n] for n in ("add", "subtract", "multiply", "divide", "maximum", "minimum")}
 _EWF_NOT = UNARY_CODES["not"]
+# evaluated in double: a result of these in fp16 takes nk_ew_f32_f16fn, which
+# narrows it in one rounding as the general kernel does
+_EWF_FUNCTIONS = {UNARY_CODES[n] for n in ("exponential", "log", "rsqrt", "tanh", "logistic")}
 EWF_RAGGED_MIN = 512 * 256  # a round of nk_ew_program: two workgroups per CU
 
 
@@ -470,7 +473,7 @@ class ProgramStep(Step):
 
 
     def _float_form(self, addr, total: int) -> Optional[Launch]:
-        """The ``nk_ew_f32`` launch, or None where a type, an operation or
+        """The ``nk_ew_f32`` (``_f16fn``) launch, or None where a type, an operation or
         an offset past 2^31 needs the general kernel."""
         p = self.prog
         if total >= 2**31 - 4096 or self.out_dtype not in _EWF_TYPES or any(
@@ -516,7 +519,9 @@ class ProgramStep(Step):
             I.op, I.dst, I.a, I.b, I.c, I.dtype, I.imm = op, dst, x, y, z, dtc, float(np.float32(imm))
         grid = max(1, min(-(-total // 1024), 65536))
         a.step = grid * 1024
-        return Launch("generic", "nk_ew_f32", (grid, 1, 1), (256, 1, 1), a, bytes=total * self.out_dtype.itemsize)
+        half = any(op in _EWF_FUNCTIONS and dtc == DT_CODE[dt.float16] for op, _, _, _, _, dtc, _, _ in p.instrs)
+        symbol = "nk_ew_f32_f16fn" if half else "nk_ew_f32"
+        return Launch("generic", symbol, (grid, 1, 1), (256, 1, 1), a, bytes=total * self.out_dtype.itemsize)
 
 
 def strided_access(v: Value, materialized) -> Tuple[Value, np.ndarray, int]:

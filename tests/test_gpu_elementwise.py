@@ -112,6 +112,37 @@ def test_ragged_rows_equal_the_general_kernel(gpu, monkeypatch, shape, d):
     assert res[0] == res[1]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", ["float16", "bfloat16"])
+def test_functions_of_every_16_bit_value(gpu, monkeypatch, d):
+    """The functions evaluated in double reach their 16-bit type in one
+    rounding: by way of fp32 about ten fp16 results (exp(0.02269), just below
+    the middle of two) fall on a tie that the true value is not on."""
+    print(f"elementwise functions {d}", flush=True)
+    bits = np.arange(65536, dtype=np.uint16).reshape(64, 1024)
+    x = dt.to_bf16((bits.astype(np.uint32) << 16).view(np.float32)) if d == "bfloat16" else bits.view(np.float16)
+
+    def fn(x):
+        return np.exp(x), np.log(x), np.sqrt(x), np.tanh(x), 1 / (1 + np.exp(-x))
+
+    res, symbols = _both(fn, [x], monkeypatch)
+    # a program a result: the roots (no function) stay on the plain kernel
+    assert "nk_ew_f32" in symbols[0] and ("nk_ew_f32_f16fn" in symbols[0]) == (d == "float16")
+    assert "nk_ew_program" not in symbols[0] and symbols[1] == {"nk_ew_program"}
+
+    def values(raw):
+        raw = np.frombuffer(raw, np.uint16).reshape(x.shape)
+        return (raw.astype(np.uint32) << 16).view(np.float32) if d == "bfloat16" else raw.view(np.float16)
+
+    for k in res[0]:
+        np.testing.assert_array_equal(values(res[0][k]), values(res[1][k]), err_msg=k)
+    if d == "float16":
+        with np.errstate(all="ignore"):
+            for k, f in zip(res[0], (np.exp, np.log, np.sqrt, np.tanh)):
+                want = f(bits.view(np.float16).astype(np.float64)).astype(np.float16)
+                np.testing.assert_array_equal(values(res[0][k]), want, err_msg=k)
+
+
 @pytest.mark.parametrize("shape,symbol", [((1000, 33), "nk_ew_program"), ((1000, 32), "nk_ew_f32"),
                                           ((3971, 33), "nk_ew_program"), ((3972, 33), "nk_ew_f32"),
                                           ((1, 33), "nk_ew_f32")])
